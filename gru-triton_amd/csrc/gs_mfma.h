@@ -395,6 +395,13 @@ inline int check_codes(const int8_t* codes, const float* scales, const char* who
     return set_error(GS_ERR_INVALID, "%s: w_codes must be 16-byte aligned", who);
   return GS_OK;
 }
+// The same recurrences with one launch per step over all CUs (scan_step.hip).
+bool step_fwd_applies(const gs_args* a);
+int run_step_fwd(const gs_args* a, hipStream_t stream, const int8_t* codes, const float* scales);
+bool step_bwd_applies(const float* dout, const float* dh0, int64_t T, int64_t B, int64_t H);
+int run_step_bwd_recurrence(const float* w, float* wt, const float* dout, const float* cg, const float* zm,
+                            const float* mi, float* dsum, float* dh0, int64_t T, int64_t B, int64_t H,
+                            hipStream_t stream);
 int64_t tiled_bwd_wt_bytes(int64_t H);
 int run_tiled_bwd_recurrence(const float* w, float* wt, const float* dout, const float* cg, const float* zm,
                              const float* mi, float* dsum, float* dh0, int64_t T, int64_t B, int64_t H,

@@ -9,9 +9,12 @@
 // requirement, no workspace and no bound on H beyond what a workgroup's LDS
 // holds. The persistent kernels (scan_dense.hip, scan_dense_bwd.hip) keep Wh
 // resident and exchange the state between workgroups every step; they are the
-// fast path up to H = 1024. These kernels serve gru_scan / gru_scan_forward by
-// name, and every dense recurrence with H > 1024 (gs_dense_fwd, gs_dense_bwd and
-// the materialized-map backwards of the structured kinds).
+// fast path up to H = 1024. Above 64 hidden units the same barrier-free contract
+// is served by one launch per step over all CUs (scan_step.hip): a step here
+// streams all of Wh through each tile's one CU, 2.9 us at H = 64 against 3.5 us
+// for a launch, but 5.7 against 3.8 at H = 128, 60 against 6 at H = 512 and 990
+// against 14.6 at H = 2048 (B = 32). These kernels run up to 64 units, and at
+// any H where a launch per step cannot: tensors that overlap (step_fwd_applies).
 //
 // Work split. A workgroup of 8 waves owns BT <= 4 batch rows. Per step each
 // wave takes quads of 4 hidden units (quad q, q + 8, ...) and forms their 3
@@ -498,6 +501,7 @@ int run_tiled_fwd(const gs_args* a, hipStream_t stream, const char* who, const i
   if (a->H > tiled_max_h())
     return set_error(GS_ERR_INVALID, "%s: hidden size %lld exceeds the supported maximum of %lld", who,
                      (long long)a->H, (long long)tiled_max_h());
+  if (step_fwd_applies(a)) return run_step_fwd(a, stream, codes, scales);
   TilePlan tp;
   int rc = plan_tiled(a->H, a->B, false, &tp, who);
   if (rc) return rc;
@@ -555,6 +559,8 @@ int run_tiled_bwd_recurrence(const float* w, float* wt, const float* dout, const
   if (H > tiled_max_h())
     return set_error(GS_ERR_INVALID, "%s: hidden size %lld exceeds the supported maximum of %lld", who,
                      (long long)H, (long long)tiled_max_h());
+  if (step_bwd_applies(dout, dh0, T, B, H))
+    return run_step_bwd_recurrence(w, wt, dout, cg, zm, mi, dsum, dh0, T, B, H, stream);
   TilePlan tp;
   int rc = plan_tiled(H, B, true, &tp, who);
   if (rc) return rc;

@@ -1,0 +1,116 @@
+"""The dense recurrences with one launch per step (scan_step.hip), which serve
+gru_scan / gru_scan_forward / gru_scan_backward_triton above 64 hidden units
+and every dense recurrence above 1024. Their products follow the persistent
+kernels' order, so up to H = 1024 both must agree bit for bit; above, the
+oracle checks of test_gpu_tiled.py apply. Sizes sit on the edges of the 16-row,
+16-unit and 64-k tiles and on each rows-per-workgroup variant."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from gru_qat_amd.configs import Q_INT8_HIDDEN, make_config
+from parity_util import log, to_dev
+
+pytestmark = pytest.mark.gpu
+
+OTHER = (0.05, -10, 10)
+# (T, B, H): 65 the smallest H; 16 / 17 and 64 / 65 rows; K one past and one short of a chunk; scalar loads
+# (H not a multiple of 4); 32 and 64 rows a workgroup (B = 60 x 1000, B = 250 x 1024)
+SHAPES = [(3, 1, 65), (4, 16, 68), (3, 17, 127), (4, 65, 129), (1, 33, 192), (3, 60, 1000), (2, 250, 1024)]
+
+
+def _cfg(shape, q_in=None, q_out=None, int8=False):
+    cfg = make_config(2 if int8 else 1, shape=shape, seed=3)
+    cfg["h_in_quant"], cfg["h_out_quant"] = q_in, q_out
+    return cfg
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("q_in,q_out", [(None, None), (Q_INT8_HIDDEN, Q_INT8_HIDDEN), (OTHER, Q_INT8_HIDDEN),
+                                        (None, OTHER)])
+def test_step_matches_persistent(dev, shape, q_in, q_out):
+    import gru_qat_amd.scan as S
+
+    cfg = _cfg(shape, q_in, q_out)
+    d = to_dev(cfg, dev)
+    T, B, H = shape
+    outs, ghs = [], []
+    for tiled in (True, False):
+        gh = torch.empty((T, B, 3 * H), device=dev)
+        outs.append(S._dense_forward("test", d["gi"], d["h0"], d["w"], d["bh"], q_in, q_out, gh_save=gh, tiled=tiled))
+        ghs.append(gh)
+    plain = S._dense_forward("test", d["gi"], d["h0"], d["w"], d["bh"], q_in, q_out, tiled=True)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(ghs[0], ghs[1]) and torch.equal(plain, outs[0])
+    dout = torch.randn(outs[0].shape, generator=torch.Generator().manual_seed(5)).to(dev)
+    a = S.gru_scan_backward_triton(d["gi"], d["h0"], d["w"], d["bh"], outs[0], dout, h_in_quant=q_in, h_out_quant=q_out)
+    b = S.gru_scan_backward_persistent(d["gi"], d["h0"], d["w"], d["bh"], outs[0], dout, h_in_quant=q_in,
+                                       h_out_quant=q_out)
+    for name, x, y in zip(("dgi", "dh0", "dWh", "dbh"), a, b):
+        assert torch.equal(x, y), name
+
+
+@pytest.mark.parametrize("shape", [(3, 1, 80), (3, 17, 272), (2, 60, 1024), (2, 33, 1040)])
+@pytest.mark.parametrize("q_out", [Q_INT8_HIDDEN, None])
+def test_step_int8_codes(dev, shape, q_out):
+    """Exact integer sums: the persistent int8 kernel's outputs up to H = 1024, and within one level of the
+    fp32 products above (a code on a rounding boundary may fall either way)."""
+    import gru_qat_amd.scan as S
+
+    cfg = _cfg(shape, Q_INT8_HIDDEN, q_out, int8=True)
+    d = to_dev(cfg, dev)
+    args = (d["gi"], d["h0"], d["w"], d["bh"], Q_INT8_HIDDEN, q_out)
+    a = S._dense_forward("test", *args, tiled=True, int8_codes=True)
+    if shape[2] <= 1024:
+        assert torch.equal(a, S._dense_forward("test", *args, int8_codes=True))
+    else:
+        err = (a - S._dense_forward("test", *args, tiled=True)).abs().max().item()
+        assert err <= 1.01 / 127, err
+
+
+def _raw(dev, name, gi, h0, w, bh, out, T, B, H, sg, so, sh0):
+    from gru_qat_amd import _lib
+
+    lib = _lib.load()
+    a = _lib.GsArgs(gi.data_ptr(), h0.data_ptr(), w.data_ptr(), None, bh.data_ptr(), out.data_ptr(), None, 0, None, T,
+                    B, H, *sg, sh0, *so, 0, 0, 0, 0, _lib.make_quant(None, "q"), _lib.make_quant(None, "q"), None)
+    rc = getattr(lib, name)(ctypes.byref(a), ctypes.c_void_p(_lib.current_stream_handle(dev)))
+    _lib.raise_for(rc, lib)
+    torch.cuda.synchronize(dev)
+
+
+@pytest.mark.parametrize("pad", [1, 4])
+def test_step_strided_and_unaligned(dev, pad):
+    """Padded rows of gi, h0 and out, and bases off 16 bytes (pad 1), give the contiguous call's outputs."""
+    T, B, H = 3, 19, 132
+    cfg = _cfg((T, B, H))
+    d = to_dev(cfg, dev)
+    ref = torch.empty((T, B, H), device=dev)
+    _raw(dev, "gs_dense_fwd_tiled", d["gi"], d["h0"], d["w"], d["bh"], ref, T, B, H, (B * 3 * H, 3 * H), (B * H, H), H)
+    gi = torch.full((T, B + 1, 3 * H + pad), float("nan"), device=dev)
+    gi[:, :B, pad:] = d["gi"]
+    h0 = torch.full((B, H + pad), float("nan"), device=dev)
+    h0[:, pad:] = d["h0"]
+    w = torch.full((3 * H * H + pad,), float("nan"), device=dev)
+    w[pad:] = d["w"].reshape(-1)
+    out = torch.full((T, B + 2, H + pad), 7.0, device=dev)
+    _raw(dev, "gs_dense_fwd_tiled", gi[0, 0, pad:], h0[0, pad:], w[pad:], d["bh"], out[0, 0, pad:], T, B, H,
+         gi.stride()[:2], out.stride()[:2], h0.stride(0))
+    assert torch.equal(out[:, :B, pad:], ref)
+    assert (out[:, :, :pad] == 7.0).all() and (out[:, B:] == 7.0).all()
+
+
+def test_step_in_place_state(dev):
+    """out on top of h0 (a streaming state updated in place) keeps running one batch tile per workgroup."""
+    T, B, H = 1, 37, 512
+    cfg = _cfg((T, B, H))
+    d = to_dev(cfg, dev)
+    ref = torch.empty((T, B, H), device=dev)
+    _raw(dev, "gs_dense_fwd_tiled", d["gi"], d["h0"], d["w"], d["bh"], ref, T, B, H, (B * 3 * H, 3 * H), (B * H, H), H)
+    state = d["h0"].clone()
+    _raw(dev, "gs_dense_fwd_tiled", d["gi"], state, d["w"], d["bh"], state, T, B, H, (B * 3 * H, 3 * H), (B * H, H), H)
+    log(f"[step] in place: {int((state != ref[0]).sum())} elements differ")
+    assert torch.equal(state, ref[0])
