@@ -31,7 +31,7 @@
 // exchange and the epilogue, about 3.3 us a step), then Wh from the caches (12
 // KiB a 64-k chunk and workgroup, 16 KiB with the state), and from a few hundred
 // rows x 1024 units the fp32 MFMA rate: at B = 256, H = 1024 a forward step's
-// products take 12.5 us at the measured 129 TFLOP/s and the step 21.3. Measured us a
+// products take 12.5 us at the measured 129 TFLOP/s and the step 19.0. Measured us a
 // step, batch-tiled -> here: forward H = 512, B = 32: 59.6 -> 5.9; H = 2048, B = 32:
 // 991 -> 14.6 (int8 codes 364 -> 8.7); whole backward per step: H = 512 37.6 -> 10.9,
 // H = 2048 556 -> 51.8 (of which the products outside the recurrence about 30).
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kStepThreads* RW, RT == 1 ? 2 : RW) void step_fwd_k
   constexpr int NB = NA + 3;                 // and one per gate of Wh
   constexpr int NL = (NB + RW - 1) / RW;     // blocks per thread
   constexpr int NO = RT + 3;                 // operands per wave
-  constexpr int PD = RW > 1 ? 1 : 4;         // even: the operand sets alternate by chunk
+  constexpr int PD = RW > 1 ? 1 : 4;         // RW 1: by_four's register sets
   constexpr bool kLateGates = RW > 1;        // no registers to hold the gate inputs across the loop
   __shared__ __attribute__((aligned(16))) float lds[2][NL * RW * 16 * kStepRS];
   static_assert(sizeof(lds) >= 4 * NA * 3 * 256 * sizeof(float), "slice sums fit the staging buffers");
@@ -699,15 +699,22 @@ int run_step_fwd(const gs_args* a, hipStream_t stream, const int8_t* codes, cons
   p.pscale = a->q_in.scale;
   const bool save = a->gh_save != nullptr;
   const int nut = (H + 15) / 16;
-  // the most rows a workgroup that still leaves about one workgroup per CU (the
-  // weights are then read by the fewest workgroups); int8 holds its level
-  // conversion in registers at up to 32
-  const int rt = !i8 && B > 32 && (int64_t)((B + 63) / 64) * nut >= 224 ? 4
-                 : B > 16 && (int64_t)((B + 31) / 32) * nut >= 224      ? 2
-                                                                         : 1;
+  // Rows a workgroup: 16, 32 or 64. A CU takes its workgroups of one kind in
+  // turn (or overlaps them, at much the same cost each): relative cost of one
+  // 64-k chunk 0.30 us for 16 rows, 0.48 for the first and 0.61 for each further
+  // workgroup of 32, 0.95 and 1.05 of 64 (H = 1024, B = 64 ... 512). int8 (its time
+  // is the level conversion, per row): 32 rows where that still fills the CUs.
+  auto rounds = [&](int r) { return (double)(((int64_t)((B + r - 1) / r) * nut + 255) / 256); };
+  int rt = 1;
+  if (i8) {
+    rt = B > 16 && (int64_t)((B + 31) / 32) * nut >= 224 ? 2 : 1;
+  } else {
+    const double c1 = 0.30 * rounds(16), c2 = 0.48 + 0.61 * (rounds(32) - 1), c4 = 0.95 + 1.05 * (rounds(64) - 1);
+    rt = c1 <= c2 && c1 <= c4 ? 1 : c2 <= c4 ? 2 : 4;
+  }
   const dim3 grid((unsigned)nut, (unsigned)((B + 16 * rt - 1) / (16 * rt)));
   typedef void (*Fn)(SFParams);
-#define GS_STEP_FWD_Q(V, S, Q) {step_fwd_kernel<1, 1, V, S, Q>, step_fwd_kernel<2, 1, V, S, Q>, step_fwd_kernel<2, 2, V, S, Q>}
+#define GS_STEP_FWD_Q(V, S, Q) {step_fwd_kernel<1, 1, V, S, Q>, step_fwd_kernel<1, 2, V, S, Q>, step_fwd_kernel<2, 2, V, S, Q>}
 #define GS_STEP_FWD(V, S) {GS_STEP_FWD_Q(V, S, false), GS_STEP_FWD_Q(V, S, true)}
   static const Fn f32[2][2][2][3] = {{GS_STEP_FWD(false, false), GS_STEP_FWD(false, true)},
                                   {GS_STEP_FWD(true, false), GS_STEP_FWD(true, true)}};
@@ -727,7 +734,7 @@ int run_step_fwd(const gs_args* a, hipStream_t stream, const int8_t* codes, cons
     const bool quant_a = a->q_in.enabled && (t == 0 || !same_quant(a->q_in, a->q_out));
     const bool vec = vec_w && H % 4 == 0 && al16(p.hprev) && (B == 1 || p.sh_b % 4 == 0);
     const Fn fn = i8 ? q8[vec ? 1 : 0][ri] : f32[vec ? 1 : 0][save ? 1 : 0][quant_a ? 1 : 0][ri];
-    hipLaunchKernelGGL(fn, grid, dim3(rt == 4 ? 2 * kStepThreads : kStepThreads), 0, stream, p);
+    hipLaunchKernelGGL(fn, grid, dim3(rt > 1 && !i8 ? 2 * kStepThreads : kStepThreads), 0, stream, p);
     GS_CHECK_HIP(hipGetLastError());
   }
   return GS_OK;
@@ -747,8 +754,13 @@ int run_step_bwd_recurrence(const float* w, float* wt, const float* dout, const 
   p.B = (int)B;
   p.H = (int)H;
   p.nch = nch;
-  auto tiles = [&](int rt, int ct) { return ((B + 16 * rt - 1) / (16 * rt)) * ((H + 16 * ct - 1) / (16 * ct)); };
-  const int sel = B > 16 && tiles(2, 2) >= 224 ? 2 : B > 16 && tiles(2, 1) >= 224 ? 1 : 0;
+  // 16 x 16, 32 x 16 or 32 x 32 (rows x units) a workgroup, by rounds of 256 workgroups; relative cost of a
+  // workgroup 6.5, 10 and 17 us at K = 3 x 1024
+  auto rounds = [&](int rt, int ct) {
+    return (double)((((B + 16 * rt - 1) / (16 * rt)) * ((H + 16 * ct - 1) / (16 * ct)) + 255) / 256);
+  };
+  const double c0 = 6.5 * rounds(1, 1), c1 = 10.0 * rounds(2, 1), c2 = 17.0 * rounds(2, 2);
+  const int sel = c0 <= c1 && c0 <= c2 ? 0 : c1 <= c2 ? 1 : 2;
   const int rt = sel >= 1 ? 2 : 1, ct = sel == 2 ? 2 : 1;
   typedef void (*Fn)(SBParams);
   static const Fn table[2][3] = {
