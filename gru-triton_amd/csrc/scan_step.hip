@@ -79,45 +79,47 @@ __device__ __forceinline__ f4 load_row4(const float* row, int k, int H) {
   return v;
 }
 
-// Operand loads of the fp32 kernels: raw buffer loads, whose per-lane offset stays
-// put while the uniform one walks K, so a chunk costs no address arithmetic;
-// the lanes past the end of a row in its last chunk, and every lane of a chunk
-// past the last, take kOffNone and read zeros without a branch.
+// Operand loads of the fp32 kernels: 16-byte raw buffer loads, whose per-lane
+// offset stays put while the uniform one walks K, so a chunk costs no address
+// arithmetic. Every lane of a chunk past the last, and the lanes that the last
+// chunk of a row does not reach, take kOffNone and read zeros without a branch.
+// gfx950 loads 16 bytes from any 4-byte address, so rows of any length and base
+// are read like this (H = 501 took 12.3 us a step with single-word loads). Only
+// where H is not a multiple of 4 (RAG) one lane of the last chunk has a row's
+// last 1 to 3 elements: it loads the row's last four instead, and fix() moves
+// them to their places. (Its offset in the chunk may then be negative, which the
+// hardware would read as past the end: row_rsrc and row_off keep 16 bytes below.)
 constexpr uint32_t kBufBytes = 0x7fffffffu;
 
-// The bits or'ed into a lane's byte offsets: 0, or kOffNone (past every row's
-// end). tail: kOffNone for the lanes that the last chunk of a row does not
-// reach. at_last / past_last (uniform): this is a row's last chunk / past it.
-__device__ __forceinline__ uint32_t off_bits(uint32_t tail, bool at_last, bool past_last) {
-  return (tail & (at_last ? ~0u : 0u)) | (past_last ? kOffNone : 0u);
+template <bool RAG>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const float* p) {
+  return bounded_rsrc(RAG ? p - 4 : p, kBufBytes);
+}
+template <bool RAG>
+__device__ __forceinline__ uint32_t row_off(int64_t elems) {
+  return 4u * (uint32_t)elems + (RAG ? 16u : 0u);
 }
 
-template <int N> struct Tail {
-  uint32_t v[N];
-};
-
-template <bool VEC>
-__device__ __forceinline__ Tail<VEC ? 1 : 4> row_tail(int klast, int H) {
-  Tail<VEC ? 1 : 4> t;
-#pragma unroll
-  for (int e = 0; e < (VEC ? 1 : 4); ++e) t.v[e] = klast + e < H ? 0u : kOffNone;
-  return t;
-}
-
-// Four floats at byte offset off + soff, with the tail bits of each load.
-template <bool VEC>
-__device__ __forceinline__ f4 buf_row4(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff,
-                                       const Tail<VEC ? 1 : 4>& bits) {
-  if constexpr (VEC) {
+template <bool RAG> struct RowTail {
+  uint32_t none;  // kOffNone for the lanes that the last chunk of a row does not reach
+  uint32_t back;  // bytes by which the lane across the row's end starts earlier in the last chunk, else 0
+  __device__ __forceinline__ RowTail(int k, int H)
+      : none(k < H ? 0u : kOffNone), back(RAG && k < H && k + 4 > H ? 4u * (k + 4 - H) : 0u) {}
+  // at_last / past_last (uniform): this is a row's last chunk / past it
+  __device__ __forceinline__ f4 load(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff, bool at_last,
+                                     bool past_last) const {
+    const uint32_t m = at_last ? ~0u : 0u;
+    if constexpr (RAG) off -= back & m;
+    off |= (none & m) | (past_last ? kOffNone : 0u);
     typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-    return __builtin_bit_cast(f4, (u4)__builtin_amdgcn_raw_buffer_load_b128(r, (int)(off | bits.v[0]), (int)soff, 0));
-  } else {
-    f4 x;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = buf_ld(r, (off + 4u * e) | bits.v[e], soff);
-    return x;
+    return __builtin_bit_cast(f4, (u4)__builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)soff, 0));
   }
-}
+  // a value loaded from a row's last chunk; rem = H % 4 (uniform, not 0)
+  __device__ __forceinline__ f4 fix(f4 x, int rem) const {
+    const f4 y = rem == 3 ? f4{x[1], x[2], x[3], 0.f} : rem == 2 ? f4{x[2], x[3], 0.f, 0.f} : f4{x[3], 0.f, 0.f, 0.f};
+    return back != 0u ? y : x;
+  }
+};
 
 // step(c, I) for c = 0 .. n - 1 with I = c mod 4 at compile time. The loop runs
 // whole groups of four and has one exit: leaving it in the middle of a group
@@ -159,7 +161,7 @@ __device__ __forceinline__ float slice_sum(const f16v& p0, const f16v& p1, int v
 // gates): RW row groups of four waves, each wave 16 RT rows. K advances in
 // chunks of 64, loaded coalesced (16 lanes a row) into PD register sets in
 // flight and staged through two LDS buffers.
-template <int RT, int RW, bool VEC, bool SAVE, bool QA>
+template <int RT, int RW, bool RAG, bool SAVE, bool QA>
 __global__ __launch_bounds__(kStepThreads* RW, RT == 1 ? 2 : RW) void step_fwd_kernel(SFParams p) {
   constexpr int NA = RT * RW;                // 16-row blocks of h
   constexpr int NB = NA + 3;                 // and one per gate of Wh
@@ -177,24 +179,22 @@ __global__ __launch_bounds__(kStepThreads* RW, RT == 1 ? 2 : RW) void step_fwd_k
   const int r16 = (tid >> 4) & 15, k4 = 4 * (tid & 15);
 
   // operand rows of this thread's loads (rows past the end repeat the last one: their products are not stored)
-  const auto rh = bounded_rsrc(p.hprev + (int64_t)row0 * p.sh_b, kBufBytes);
-  const auto rwt = bounded_rsrc(p.w, kBufBytes);
+  const auto rh = row_rsrc<RAG>(p.hprev + (int64_t)row0 * p.sh_b);
+  const auto rwt = row_rsrc<RAG>(p.w);
   const int last = p.nch - 1;
   uint32_t off[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int blk = i * RW + rw;
-    off[i] = 4u * (uint32_t)((blk < NA ? (int64_t)min(16 * blk + r16, p.B - 1 - row0) * p.sh_b
-                                       : ((int64_t)min(blk - NA, 2) * H + min(u0 + r16, H - 1)) * H) +
-                             k4);
+    off[i] = row_off<RAG>((blk < NA ? (int64_t)min(16 * blk + r16, p.B - 1 - row0) * p.sh_b
+                                    : ((int64_t)min(blk - NA, 2) * H + min(u0 + r16, H - 1)) * H) +
+                          k4);
   }
-  const auto tail = row_tail<VEC>(64 * last + k4, H);
+  const RowTail<RAG> tail(64 * last + k4, H);
   f4 reg[PD][NL];
   auto load = [&](int c, f4 (&x)[NL]) __attribute__((always_inline)) {
-    auto bits = tail;
-    for (auto& v : bits.v) v = off_bits(v, c == last, c > last);
 #pragma unroll
-    for (int i = 0; i < NL; ++i) x[i] = buf_row4<VEC>(i * RW + rw < NA ? rh : rwt, off[i], 256u * c, bits);
+    for (int i = 0; i < NL; ++i) x[i] = tail.load(i * RW + rw < NA ? rh : rwt, off[i], 256u * c, c == last, c > last);
   };
   static_for<0, PD>([&](auto I) { load(I, reg[I]); });
 
@@ -229,6 +229,10 @@ __global__ __launch_bounds__(kStepThreads* RW, RT == 1 ? 2 : RW) void step_fwd_k
   const int rd = (lane & 15) * kStepRS + 16 * wave + 4 * (lane >> 4);
   auto write = [&](int c, f4 (&x)[NL]) __attribute__((always_inline)) {
     float* buf = lds[c & 1];
+    if (RAG && c == last) {  // uniform
+#pragma unroll
+      for (int i = 0; i < NL; ++i) x[i] = tail.fix(x[i], H & 3);
+    }
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int blk = i * RW + rw;
@@ -274,7 +278,7 @@ __global__ __launch_bounds__(kStepThreads* RW, RT == 1 ? 2 : RW) void step_fwd_k
       write(c + 2, reg[(I + 2) % PD]);
       load(c + 2 + PD, reg[(I + 2) % PD]);
       mfma(o[I & 1]);
-      interleave<12 * RT, NO, NL, VEC ? NL : 4 * NL>();
+      interleave<12 * RT, NO, NL, NL>();
       lds_barrier();
     };
     by_four(p.nch, step);
@@ -289,7 +293,7 @@ __global__ __launch_bounds__(kStepThreads* RW, RT == 1 ? 2 : RW) void step_fwd_k
       write(c + 1, reg[0]);
       load(c + 2, reg[0]);
       mfma(o);
-      interleave<12 * RT, NO, NL, VEC ? NL : 4 * NL>();
+      interleave<12 * RT, NO, NL, NL>();
       lds_barrier();
     }
   }
@@ -477,7 +481,7 @@ struct SBParams {
   int B, H, nch, last;  // last: t = 0
 };
 
-template <int RT, int CT, bool VEC>
+template <int RT, int CT, bool RAG>
 __global__ __launch_bounds__(kStepThreads) void step_bwd_kernel(SBParams p) {
   constexpr int NP = RT + CT;
   constexpr int QS = RT * CT == 1 ? 2 : 1;  // 64-chunks per stage
@@ -491,19 +495,20 @@ __global__ __launch_bounds__(kStepThreads) void step_bwd_kernel(SBParams p) {
   const int r16 = tid >> 4, k4 = 4 * (tid & 15);
   const int ldw = 64 * nk;
 
-  const auto rd_ = bounded_rsrc(p.d + (int64_t)row0 * H, kBufBytes);
-  const auto rc_ = bounded_rsrc(p.cg + (int64_t)row0 * 3 * H, kBufBytes);
-  const auto rw_ = bounded_rsrc(p.wt, kBufBytes);
+  const auto rd_ = row_rsrc<RAG>(p.d + (int64_t)row0 * H);
+  const auto rc_ = row_rsrc<RAG>(p.cg + (int64_t)row0 * 3 * H);
+  const auto rw_ = row_rsrc<false>(p.wt);
   uint32_t offd[RT], offc[RT], offw[CT];
 #pragma unroll
   for (int i = 0; i < RT; ++i) {
     const uint32_t row = min(16 * i + r16, p.B - 1 - row0);
-    offd[i] = 4u * (row * H + k4);
-    offc[i] = 4u * (row * 3 * H + k4);
+    offd[i] = row_off<RAG>(row * H + k4);
+    offc[i] = row_off<RAG>(row * 3 * H + k4);
   }
 #pragma unroll
-  for (int j = 0; j < CT; ++j) offw[j] = 4u * ((uint32_t)min(u0 + 16 * j + r16, H - 1) * ldw + k4);
-  const auto tail = row_tail<VEC>(64 * (p.nch - 1) + k4, H);
+  for (int j = 0; j < CT; ++j) offw[j] = row_off<false>((int64_t)min(u0 + 16 * j + r16, H - 1) * ldw + k4);
+  const RowTail<RAG> tail(64 * (p.nch - 1) + k4, H);
+  const RowTail<false> whole(0, 64);  // wt's rows are padded to whole chunks
   struct Set {
     f4 d[QS][RT], c[QS][RT], w[QS][CT];
   };
@@ -515,16 +520,14 @@ __global__ __launch_bounds__(kStepThreads) void step_bwd_kernel(SBParams p) {
       const int cc = s * QS + q;
       const int g = cc >= 2 * p.nch ? 2 : cc >= p.nch ? 1 : 0;
       const int kc = cc - g * p.nch;  // chunk of the gate
-      auto bits = tail;
-      for (auto& v : bits.v) v = off_bits(v, kc == p.nch - 1, cc >= nk);
+      const bool at_last = kc == p.nch - 1, past = cc >= nk;
 #pragma unroll
       for (int i = 0; i < RT; ++i) {
-        x.d[q][i] = buf_row4<VEC>(rd_, offd[i], 256u * kc, bits);
-        x.c[q][i] = buf_row4<VEC>(rc_, offc[i], 256u * kc + 4u * g * H, bits);
+        x.d[q][i] = tail.load(rd_, offd[i], 256u * kc, at_last, past);
+        x.c[q][i] = tail.load(rc_, offc[i], 256u * kc + 4u * g * H, at_last, past);
       }
-      const Tail<1> none{{off_bits(0u, false, cc >= nk)}};
 #pragma unroll
-      for (int j = 0; j < CT; ++j) x.w[q][j] = buf_row4<true>(rw_, offw[j], 256u * cc, none);
+      for (int j = 0; j < CT; ++j) x.w[q][j] = whole.load(rw_, offw[j], 256u * cc, false, past);
     }
   };
   static_for<0, PD>([&](auto I) { load(I, reg[I]); });
@@ -558,6 +561,16 @@ __global__ __launch_bounds__(kStepThreads) void step_bwd_kernel(SBParams p) {
     float* buf = lds[s & 1];
 #pragma unroll
     for (int q = 0; q < QS; ++q) {
+      if (RAG) {
+        const int cc = s * QS + q;
+        if (cc == p.nch - 1 || cc == 2 * p.nch - 1 || cc == nk - 1) {  // a gate's last chunk (uniform)
+#pragma unroll
+          for (int i = 0; i < RT; ++i) {
+            x.d[q][i] = tail.fix(x.d[q][i], H & 3);
+            x.c[q][i] = tail.fix(x.c[q][i], H & 3);
+          }
+        }
+      }
 #pragma unroll
       for (int i = 0; i < RT; ++i) *reinterpret_cast<f4*>(buf + i * 16 * RS + st + 64 * q) = x.d[q][i] * x.c[q][i];
 #pragma unroll
@@ -714,16 +727,14 @@ int run_step_fwd(const gs_args* a, hipStream_t stream, const int8_t* codes, cons
   }
   const dim3 grid((unsigned)nut, (unsigned)((B + 16 * rt - 1) / (16 * rt)));
   typedef void (*Fn)(SFParams);
-#define GS_STEP_FWD_Q(V, S, Q) {step_fwd_kernel<1, 1, V, S, Q>, step_fwd_kernel<1, 2, V, S, Q>, step_fwd_kernel<2, 2, V, S, Q>}
-#define GS_STEP_FWD(V, S) {GS_STEP_FWD_Q(V, S, false), GS_STEP_FWD_Q(V, S, true)}
+#define GS_STEP_FWD_Q(R, S, Q) {step_fwd_kernel<1, 1, R, S, Q>, step_fwd_kernel<1, 2, R, S, Q>, step_fwd_kernel<2, 2, R, S, Q>}
+#define GS_STEP_FWD(R, S) {GS_STEP_FWD_Q(R, S, false), GS_STEP_FWD_Q(R, S, true)}
   static const Fn f32[2][2][2][3] = {{GS_STEP_FWD(false, false), GS_STEP_FWD(false, true)},
                                   {GS_STEP_FWD(true, false), GS_STEP_FWD(true, true)}};
 #undef GS_STEP_FWD
 #undef GS_STEP_FWD_Q
   static const Fn q8[2][2] = {{step_fwd_i8_kernel<1, false>, step_fwd_i8_kernel<2, false>},
                               {step_fwd_i8_kernel<1, true>, step_fwd_i8_kernel<2, true>}};
-  // 16-byte loads of Wh (or its codes: aligned by contract) and of the state rows
-  const bool vec_w = i8 || (H % 4 == 0 && al16(a->w));
   const int ri = rt == 4 ? 2 : rt == 2 ? 1 : 0;
   for (int64_t t = 0; t < a->T; ++t) {
     p.gi = a->gi + t * a->sg_t;
@@ -732,8 +743,8 @@ int run_step_fwd(const gs_args* a, hipStream_t stream, const int8_t* codes, cons
     p.out = a->out + t * a->so_t;
     p.gh_save = save ? a->gh_save + t * B * 3 * H : nullptr;
     const bool quant_a = a->q_in.enabled && (t == 0 || !same_quant(a->q_in, a->q_out));
-    const bool vec = vec_w && H % 4 == 0 && al16(p.hprev) && (B == 1 || p.sh_b % 4 == 0);
-    const Fn fn = i8 ? q8[vec ? 1 : 0][ri] : f32[vec ? 1 : 0][save ? 1 : 0][quant_a ? 1 : 0][ri];
+    const bool vec = al16(p.hprev) && (B == 1 || p.sh_b % 4 == 0);
+    const Fn fn = i8 ? q8[vec ? 1 : 0][ri] : f32[H % 4 != 0 ? 1 : 0][save ? 1 : 0][quant_a ? 1 : 0][ri];
     hipLaunchKernelGGL(fn, grid, dim3(rt > 1 && !i8 ? 2 * kStepThreads : kStepThreads), 0, stream, p);
     GS_CHECK_HIP(hipGetLastError());
   }
@@ -777,8 +788,7 @@ int run_step_bwd_recurrence(const float* w, float* wt, const float* dout, const 
     p.dst = t > 0 ? dsum + (t - 1) * BH : dh0;
     p.dfirst = first ? dsum + t * BH : nullptr;
     p.last = t == 0;
-    const bool vec = H % 4 == 0 && al16(p.d);
-    hipLaunchKernelGGL(table[vec ? 1 : 0][sel], grid, dim3(kStepThreads), 0, stream, p);
+    hipLaunchKernelGGL(table[H % 4 != 0 ? 1 : 0][sel], grid, dim3(kStepThreads), 0, stream, p);
     GS_CHECK_HIP(hipGetLastError());
   }
   return GS_OK;
