@@ -375,9 +375,11 @@ BFn pick_bwd(int KC, int* nt) {
 // Workspace (tagged words only): control words | xh [2][Bp][H] tagged D |
 // xw [nrb P]. Scratch (plain floats), each region 256-byte aligned:
 // cg [T B, 3H] | hq, cgn, zm, mi, dsum [T B, H] each |
-// dbh chunks [nchunks][B][3H] | dWh split partials.
+// dbh chunks [nchunks][B][3H] | dWh split partials | Wh transposed (batch-tiled
+// kernel, launch per step).
 struct BPlan {
-  bool tiled;  // the recurrence runs on the batch-tiled kernel (scan_tiled.hip)
+  bool tiled;  // the recurrence runs on the batch-tiled kernel (scan_tiled.hip) or a launch per step
+  bool step;   // it would run on the persistent kernel, but a launch per step is faster (scan_step.hip)
   int KC, nt, nwc, P, nrb, Bp, hsz, split, nchunks;
   int64_t xh_bytes, xw_bytes, cg_bytes, plane_bytes, chunk_bytes, part_bytes, wt_bytes;
   int64_t total() const { return tiled ? 0 : kCtrlBytes + xh_bytes + xw_bytes; }
@@ -389,6 +391,7 @@ struct BPlan {
 int plan_bwd(const gs_bwd_args* a, BPlan* pl, const char* who, bool tiled) {
   const int H = (int)a->H;
   pl->tiled = tiled || a->H > kPersistentMaxH;
+  pl->step = !pl->tiled && step_bwd_beats_persistent(a->B, a->H);  // by shape alone: size queries have no tensors yet
   pl->KC = pl->nt = pl->nwc = pl->P = pl->hsz = 0;
   pl->xh_bytes = pl->xw_bytes = pl->wt_bytes = 0;
   pl->nrb = (int)((a->B + 3) / 4);
@@ -399,6 +402,7 @@ int plan_bwd(const gs_bwd_args* a, BPlan* pl, const char* who, bool tiled) {
                        (long long)tiled_max_h());
     pl->wt_bytes = tiled_bwd_wt_bytes(H);
   } else {
+    if (pl->step) pl->wt_bytes = tiled_bwd_wt_bytes(H);
     pl->KC = choose_kc(H);
     if (pl->KC < 0)
       return set_error(GS_ERR_INVALID, "%s: hidden size %d exceeds the supported maximum of 1024", who, H);
@@ -567,6 +571,10 @@ int dense_bwd_core(const gs_bwd_args* a, const float* w, float* dw, hipStream_t 
   if (pl.tiled) {
     float* wt = reinterpret_cast<float*>(take(pl.wt_bytes));
     rc = run_tiled_bwd_recurrence(w, wt, a->dout, cg, zm, mi, dsum, a->dh0, T, B, H, stream, who);
+    if (rc) return rc;
+  } else if (pl.step && step_bwd_applies(a->dout, a->dh0, T, B, H)) {
+    float* wt = reinterpret_cast<float*>(take(pl.wt_bytes));
+    rc = run_step_bwd_recurrence(w, wt, a->dout, cg, zm, mi, dsum, a->dh0, T, B, H, stream);
     if (rc) return rc;
   } else {
     rc = launch_recurrence(pl, w, a, cg, zm, mi, dsum, xh, xw, ws, stream, who);

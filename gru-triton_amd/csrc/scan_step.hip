@@ -688,6 +688,40 @@ bool step_fwd_applies(const gs_args* a) {
          !overlap(a->out, n_out, a->w, 3 * a->H * a->H);
 }
 
+namespace {
+// 4-row blocks that a group of the persistent dense kernels takes in turn: P
+// workgroups of 16 units (48 below KC 16) a group, one workgroup per CU.
+int64_t persistent_rounds(int64_t B, int64_t H, int kc) {
+  const int64_t upw = kc >= 16 ? 16 : 48;
+  const int64_t groups = std::max<int64_t>(1, 256 / ((H + upw - 1) / upw));
+  return ((B + 3) / 4 + groups - 1) / groups;
+}
+}  // namespace
+
+// The persistent kernels take about 1.15 us (H <= 256), 1.5 (<= 512) or 2.8 (<=
+// 1024) a round, int8 codes 0.8, 1.1 or 1.0; a step here 4 to 8 us plus its
+// products. Measured, us a step, persistent / here: fp32 H = 256, B = 256 (4
+// rounds) 4.6 / 4.8, B = 384 (6) 6.7 / 5.5; H = 384, B = 160 (4) 6.9 / 5.3;
+// H = 512, B = 96 (3) 4.7 / 5.7, B = 256 (8) 12.0 / 7.7; H = 640, B = 48 (2) 6.1 / 6.2;
+// H = 1024, B = 48 (3) 8.7 / 8.0, B = 256 (16) 44.3 / 19.6. int8 H = 256, B = 384 (6)
+// 4.5 / 4.4; H = 384, B = 160 (4) 5.1 / 4.1; H = 768, B = 96 (5) 5.9 / 6.5, B = 160 (8) 8.6 /
+// 6.5; H = 1024, B = 160 (10) 9.7 / 11.3, B = 256 (16) 15.2 / 11.7.
+bool step_fwd_beats_persistent(const gs_args* a, bool i8) {
+  const int kc = a->H <= kPersistentMaxH ? choose_kc((int)a->H) : 0;
+  const int64_t rounds = kc < 16 ? 0 : persistent_rounds(a->B, a->H, kc);
+  const int64_t least = i8 ? (kc == 16 ? 7 : kc == 32 ? 4 : a->H <= 768 ? 7 : 12) : kc == 16 ? 6 : kc == 32 ? 4 : 3;
+  return kc >= 16 && rounds >= least && step_fwd_applies(a);
+}
+
+// The whole backward, us a step, persistent / here: H = 256, B = 384 (6 rounds)
+// 14.4 / 14.2, B = 512 (8) 18.4 / 16.3; H = 512, B = 160 (5) 17.1 / 18.4, B = 256 (8)
+// 27 / 23; H = 1024, B = 32 (2) 17.2 / 18.4, B = 48 (3) 24.1 / 20.6, B = 256 (16) 122 / 63.
+bool step_bwd_beats_persistent(int64_t B, int64_t H) {
+  const int kc = H <= kPersistentMaxH ? choose_kc((int)H) : 0;
+  const int64_t least = kc == 16 ? 7 : kc == 32 ? 7 : 3;
+  return kc >= 16 && B <= kStepMaxB && persistent_rounds(B, H, kc) >= least;
+}
+
 // dh0 is written by the launch that reads D_0, and dout is D_{T-1}.
 bool step_bwd_applies(const float* dout, const float* dh0, int64_t T, int64_t B, int64_t H) {
   return H >= kStepMinH && B <= kStepMaxB && !overlap(dh0, B * H, dout, T * B * H);

@@ -71,6 +71,36 @@ def test_step_int8_codes(dev, shape, q_out):
         assert err <= 1.01 / 127, err
 
 
+@pytest.mark.parametrize("shape", [(3, 48, 1000), (2, 97, 640), (2, 250, 501), (2, 260, 320)])
+@pytest.mark.parametrize("q", [None, Q_INT8_HIDDEN])
+def test_large_batches_on_the_persistent_entries(dev, shape, q):
+    """gru_scan_persistent's batches that run with a launch per step: every row equals the same row of a
+    batch small enough for the persistent kernel, forward (fp32 and int8 codes), gh and gradients."""
+    import gru_qat_amd.scan as S
+
+    cfg = _cfg(shape, q, q, int8=q is not None)
+    d = to_dev(cfg, dev)
+    T, B, H = shape
+    n = 5
+
+    def run(gi, h0, dout, codes):
+        gh = None if codes else torch.empty((T, gi.shape[1], 3 * H), device=dev)
+        out = S._dense_forward("test", gi, h0, d["w"], d["bh"], q, q, gh_save=gh, int8_codes=codes)
+        if codes:
+            return [out]
+        g = S._dense_backward("test", gi, h0, d["w"], d["bh"], out, dout, q, q, gh_saved=gh)
+        return [out, gh, g[0], g[1][None]]
+
+    dout = torch.randn((T, B, H), generator=torch.Generator().manual_seed(5)).to(dev)
+    for codes in (False, True) if q is not None and H % 16 == 0 else (False,):
+        whole = run(d["gi"], d["h0"], dout, codes)
+        for lo in (0, B - n):
+            rows = slice(lo, lo + n)
+            part = run(d["gi"][:, rows].contiguous(), d["h0"][rows].contiguous(), dout[:, rows].contiguous(), codes)
+            for x, y in zip(whole, part):
+                assert torch.equal(x[:, rows], y), (codes, lo)
+
+
 def _raw(dev, name, gi, h0, w, bh, out, T, B, H, sg, so, sh0):
     from gru_qat_amd import _lib
 
