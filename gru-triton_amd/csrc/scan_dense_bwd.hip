@@ -391,7 +391,7 @@ struct BPlan {
 int plan_bwd(const gs_bwd_args* a, BPlan* pl, const char* who, bool tiled) {
   const int H = (int)a->H;
   pl->tiled = tiled || a->H > kPersistentMaxH;
-  pl->step = !pl->tiled && step_bwd_beats_persistent(a->B, a->H);  // by shape alone: size queries have no tensors yet
+  pl->step = !pl->tiled && step_bwd_beats_persistent(a->T, a->B, a->H);  // by shape alone: size queries have no tensors yet
   pl->KC = pl->nt = pl->nwc = pl->P = pl->hsz = 0;
   pl->xh_bytes = pl->xw_bytes = pl->wt_bytes = 0;
   pl->nrb = (int)((a->B + 3) / 4);

@@ -667,10 +667,11 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 bool overlap(const float* a, int64_t an, const float* b, int64_t bn) { return a < b + bn && b < a + an; }
 
 // Smallest H that takes a launch per step: below, a batch tile's step on one CU
-// (scan_tiled.hip) is shorter than a launch. B = 32, T = 64, us a step, one CU
-// against a launch: forward 1.2 / 3.4 at H = 16, 2.9 / 3.6 at 64, 4.5 / 3.6 at
-// 96; backward (all its passes) 3.5 / 4.6 at 64, 5.3 / 4.9 at 96.
-constexpr int64_t kStepMinH = 65;
+// (scan_tiled.hip) is not longer than a launch on the GPU and its 2.5 us on the
+// host. B = 32, T = 64, us a step, one CU against a launch: forward 2.9 / 3.6 at
+// H = 64, 5.7 / 3.8 at 128, 12.2 / 4.1 at 192; backward (all its passes) 3.5 / 4.6 at 64,
+// 6.4 / 5.0 at 128, 9.7 / 6.2 at 192.
+constexpr int64_t kStepMinH = 129;
 constexpr int64_t kStepMaxB = 16 * 65535;  // 16-row tiles in the grid's second dimension
 
 }  // namespace
@@ -696,6 +697,9 @@ int64_t persistent_rounds(int64_t B, int64_t H, int kc) {
   const int64_t groups = std::max<int64_t>(1, 256 / ((H + upw - 1) / upw));
   return ((B + 3) / 4 + groups - 1) / groups;
 }
+// T launches cost the host 2.5 us each, which shows while the whole recurrence
+// is only some 50 us of a call that the host bounds.
+bool pays_launches(int64_t T, int64_t rounds) { return T == 1 || T * rounds >= 32; }
 }  // namespace
 
 // The persistent kernels take about 1.15 us (H <= 256), 1.5 (<= 512) or 2.8 (<=
@@ -710,21 +714,26 @@ bool step_fwd_beats_persistent(const gs_args* a, bool i8) {
   const int kc = a->H <= kPersistentMaxH ? choose_kc((int)a->H) : 0;
   const int64_t rounds = kc < 16 ? 0 : persistent_rounds(a->B, a->H, kc);
   const int64_t least = i8 ? (kc == 16 ? 7 : kc == 32 ? 4 : a->H <= 768 ? 7 : 12) : kc == 16 ? 6 : kc == 32 ? 4 : 3;
-  return kc >= 16 && rounds >= least && step_fwd_applies(a);
+  return kc >= 16 && rounds >= least && pays_launches(a->T, rounds) && step_fwd_applies(a);
 }
 
 // The whole backward, us a step, persistent / here: H = 256, B = 384 (6 rounds)
 // 14.4 / 14.2, B = 512 (8) 18.4 / 16.3; H = 512, B = 160 (5) 17.1 / 18.4, B = 256 (8)
 // 27 / 23; H = 1024, B = 32 (2) 17.2 / 18.4, B = 48 (3) 24.1 / 20.6, B = 256 (16) 122 / 63.
-bool step_bwd_beats_persistent(int64_t B, int64_t H) {
+bool step_bwd_beats_persistent(int64_t T, int64_t B, int64_t H) {
   const int kc = H <= kPersistentMaxH ? choose_kc((int)H) : 0;
   const int64_t least = kc == 16 ? 7 : kc == 32 ? 7 : 3;
-  return kc >= 16 && B <= kStepMaxB && persistent_rounds(B, H, kc) >= least;
+  const int64_t rounds = kc < 16 ? 0 : persistent_rounds(B, H, kc);
+  return kc >= 16 && B <= kStepMaxB && rounds >= least && pays_launches(T, rounds);
 }
 
-// dh0 is written by the launch that reads D_0, and dout is D_{T-1}.
+// dh0 is written by the launch that reads D_0, and dout is D_{T-1}. A few steps
+// of few units are over before the host has queued a launch each (T = 3, B = 5,
+// H = 66, a training step that the host bounds: 152 us with the one-CU kernel,
+// 162 with launches), so two steps or more take launches from T H^2 = 200000
+// on (about 30 us of the one-CU kernel).
 bool step_bwd_applies(const float* dout, const float* dh0, int64_t T, int64_t B, int64_t H) {
-  return H >= kStepMinH && B <= kStepMaxB && !overlap(dh0, B * H, dout, T * B * H);
+  return H >= kStepMinH && B <= kStepMaxB && (T == 1 || T * H * H >= 200000) && !overlap(dh0, B * H, dout, T * B * H);
 }
 
 // The forward, one launch per step (see the header comment).

@@ -9,12 +9,13 @@
 // requirement, no workspace and no bound on H beyond what a workgroup's LDS
 // holds. The persistent kernels (scan_dense.hip, scan_dense_bwd.hip) keep Wh
 // resident and exchange the state between workgroups every step; they are the
-// fast path up to H = 1024. Above 64 hidden units the same barrier-free contract
+// fast path up to H = 1024. Above 128 hidden units the same barrier-free contract
 // is served by one launch per step over all CUs (scan_step.hip): a step here
-// streams all of Wh through each tile's one CU, 2.9 us at H = 64 against 3.5 us
-// for a launch, but 5.7 against 3.8 at H = 128, 60 against 6 at H = 512 and 990
-// against 14.6 at H = 2048 (B = 32). These kernels run up to 64 units, and at
-// any H where a launch per step cannot: tensors that overlap (step_fwd_applies).
+// streams all of Wh through each tile's one CU, 2.9 us at H = 64 against 3.6 us
+// for a launch, but 12 against 4 at H = 192, 60 against 6 at H = 512 and 990
+// against 14.6 at H = 2048 (B = 32). These kernels run up to 128 units, in the
+// backward also a few steps of a few hundred, and at any H where a launch per
+// step cannot: tensors that overlap (step_fwd_applies, step_bwd_applies).
 //
 // Work split. A workgroup of 8 waves owns BT <= 4 batch rows. Per step each
 // wave takes quads of 4 hidden units (quad q, q + 8, ...) and forms their 3

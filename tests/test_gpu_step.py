@@ -1,5 +1,5 @@
 """The dense recurrences with one launch per step (scan_step.hip), which serve
-gru_scan / gru_scan_forward / gru_scan_backward_triton above 64 hidden units
+gru_scan / gru_scan_forward / gru_scan_backward_triton above 128 hidden units
 and every dense recurrence above 1024. Their products follow the persistent
 kernels' order, so up to H = 1024 both must agree bit for bit; above, the
 oracle checks of test_gpu_tiled.py apply. Sizes sit on the edges of the 16-row,
@@ -18,9 +18,10 @@ from parity_util import log, to_dev
 pytestmark = pytest.mark.gpu
 
 OTHER = (0.05, -10, 10)
-# (T, B, H): 65 the smallest H; 16 / 17 and 64 / 65 rows; K one past and one short of a chunk; scalar loads
-# (H not a multiple of 4); 32 and 64 rows a workgroup (B = 60 x 1000, B = 250 x 1024)
-SHAPES = [(3, 1, 65), (4, 16, 68), (3, 17, 127), (4, 65, 129), (1, 33, 192), (3, 60, 1000), (2, 250, 1024)]
+# (T, B, H): 129 the smallest H; 16 / 17 and 64 / 65 rows; K one past and one short of a chunk; rows of every
+# length modulo 4; T H^2 on both sides of the backward's bound; 32 and 64 rows a workgroup (B = 90 x 1000,
+# B = 250 x 1024)
+SHAPES = [(13, 1, 129), (11, 16, 130), (3, 17, 191), (4, 65, 257), (1, 33, 192), (3, 90, 1000), (2, 250, 1024)]
 
 
 def _cfg(shape, q_in=None, q_out=None, int8=False):
@@ -53,7 +54,7 @@ def test_step_matches_persistent(dev, shape, q_in, q_out):
         assert torch.equal(x, y), name
 
 
-@pytest.mark.parametrize("shape", [(3, 1, 80), (3, 17, 272), (2, 60, 1024), (2, 33, 1040)])
+@pytest.mark.parametrize("shape", [(3, 1, 144), (3, 17, 272), (2, 60, 1024), (2, 33, 1040)])
 @pytest.mark.parametrize("q_out", [Q_INT8_HIDDEN, None])
 def test_step_int8_codes(dev, shape, q_out):
     """Exact integer sums: the persistent int8 kernel's outputs up to H = 1024, and within one level of the
@@ -71,7 +72,7 @@ def test_step_int8_codes(dev, shape, q_out):
         assert err <= 1.01 / 127, err
 
 
-@pytest.mark.parametrize("shape", [(3, 48, 1000), (2, 97, 640), (2, 250, 501), (2, 260, 320)])
+@pytest.mark.parametrize("shape", [(11, 48, 1000), (8, 97, 640), (4, 250, 501), (1, 260, 320)])
 @pytest.mark.parametrize("q", [None, Q_INT8_HIDDEN])
 def test_large_batches_on_the_persistent_entries(dev, shape, q):
     """gru_scan_persistent's batches that run with a launch per step: every row equals the same row of a
@@ -115,7 +116,7 @@ def _raw(dev, name, gi, h0, w, bh, out, T, B, H, sg, so, sh0):
 @pytest.mark.parametrize("pad", [1, 4])
 def test_step_strided_and_unaligned(dev, pad):
     """Padded rows of gi, h0 and out, and bases off 16 bytes (pad 1), give the contiguous call's outputs."""
-    T, B, H = 3, 19, 132
+    T, B, H = 3, 19, 146
     cfg = _cfg((T, B, H))
     d = to_dev(cfg, dev)
     ref = torch.empty((T, B, H), device=dev)
