@@ -13,20 +13,22 @@
 //
 // A quantizer's scale depends on the min and max of the whole tensor it sees,
 // so every step has a grid-wide reduction between computing h_t and
-// quantizing it. The steps therefore run as short launches on the stream, with
+// quantizing it. The steps therefore run as one launch each on the stream, with
 // all scales kept on the device:
 //   once:      the map as a dense [3H, H] matrix (gs_hidden_map_dense) unless
-//              the kind is dense or diagonal; q_in's statistics of h0; hq_0.
-//   per step:  gh = hq W^T + bh (MFMA GEMM, K-split partials; the diagonal kind
-//              folds w_g * hq into the next kernel), the gates with a (min,
-//              max) partial per workgroup (pre-quant h_t goes to out[t]), one
-//              workgroup that reduces the partials and updates the scales and
-//              statistics, and an elementwise pass that applies q_out to out[t]
-//              in place and q_in for the next step's hq.
-// fq is monotone, so the min and max of q_out(h_t), which q_in sees at step
-// t + 1, are q_out of the pre-quant min and max: one reduction per step covers
+//              the kind is dense or diagonal; (min, max) partials of h0.
+//   step t:    every workgroup reduces the partials of the pre-quant h_{t-1}
+//              itself and derives q_out's and q_in's scales (workgroup 0 alone
+//              updates the statistics and the trace), applies both to the rows
+//              it multiplies, and runs the product, the gates and the (min, max)
+//              partial of its part of the pre-quant h_t. out[t-1] = q_out(h_{t-1})
+//              is written on the way by the workgroup that owns the element.
+//   at last:   out[T-1] = q_out(h_{T-1}).
+// fq is monotone, so the min and max of q_out(h_{t-1}), which q_in sees at step
+// t, are q_out of the pre-quant min and max: one reduction per step covers
 // both quantizers.
 #include "gs_gemm.h"
+#include "gs_mfma.h"
 
 namespace gs {
 
@@ -38,7 +40,7 @@ namespace {
 
 constexpr int kRedThreads = 256;
 constexpr int kMaxParts = 512;  // (min, max) partials of one reduction
-constexpr int kMaxSplit = 8;    // K splits of the per-step GEMM
+constexpr int kMaxSplit = 8;    // K splits of a step's product, one wave each
 // _update_observer's mixing weights as the fp32 values torch multiplies by.
 constexpr float kKeep = (float)0.99;
 constexpr float kMix = (float)(1.0 - 0.99);
@@ -223,49 +225,375 @@ __global__ __launch_bounds__(kRedThreads) void quant_step(const float2* part, in
   }
 }
 
-// The gates of one step; writes the pre-quant h_t to out_t and a (min, max)
-// partial per workgroup. gh comes from `nsplit` GEMM partials [B, 3H] (split 0
-// holds the bias), or, for the diagonal kind (dw != null), is dw_g * hq + bh_g.
-__global__ __launch_bounds__(kRedThreads) void gates_step(const float* gi_t, int64_t sg_b, const float* gh, int nsplit,
-                                                          int64_t split_stride, const float* dw, const float* bh,
-                                                          const float* hq, int64_t shq_b, const float* hprev,
-                                                          int64_t shp_b, float* out_t, int64_t so_b, int B, int H,
-                                                          float2* part) {
-  float mn = __builtin_inff(), mx = -__builtin_inff();
-  const int64_t n = (int64_t)B * H;
-  for (int64_t e = blockIdx.x * (int64_t)kRedThreads + threadIdx.x; e < n; e += (int64_t)gridDim.x * kRedThreads) {
-    const int b = (int)(e / H), k = (int)(e - (int64_t)b * H);
-    float g3[3];
-    if (dw != nullptr) {
-      const float h = hq[(int64_t)b * shq_b + k];
-#pragma unroll
-      for (int g = 0; g < 3; ++g) {
+// ---- one step ------------------------------------------------------------------------
+
+// fq at a scale found at run time. A symmetric one in quant_code's range takes
+// its division-free quotient, which equals the IEEE one (gs_device.h).
+struct DynQuant {
+  Quant q;
+  float zp;
+  int on, fast;
+  __device__ __forceinline__ float operator()(float x) const {
 #pragma clang fp contract(off)
-        g3[g] = dw[g * H + k] * h + bh[g * H + k];
-      }
-    } else {
-      const float* p = gh + (int64_t)b * 3 * H + k;
-      float v[kMaxSplit][3];
+    if (fast) {
+      float v = quant_code(x, q);
+      v = __builtin_fminf(__builtin_fmaxf(v, q.qmin), q.qmax);
+      return v * q.scale;
+    }
+    return on ? fq(x, q.scale, zp, q.qmin, q.qmax) : x;
+  }
+};
+
+__device__ __forceinline__ DynQuant dyn_quant(const Obs& o, float s, float zp) {
+  DynQuant d{{s, o.qmin, o.qmax, 1, 1.0f / s}, zp, o.mode != GS_OBS_OFF, 0};
+  d.fast = d.on && zp == 0.0f && s >= 0x1p-126f && s <= 0x1p64f;
+  return d;
+}
+
+struct OStep {
+  const float* gi;     // of step t
+  const float* hprev;  // pre-quant h_{t-1}, or h0
+  const float* w;      // the map [3H, H], or the diagonal kind's [3, H]
+  const float* bh;
+  float* hnext;        // pre-quant h_t
+  float* out_prev;     // out[t-1], or NULL at t = 0
+  const float2* part_in;
+  float2* part_out;
+  float* st;     // the scale and zero point of q_in at step t (written here; read for step t - 1's trace)
+  float* trace;  // of step t - 1, or NULL
+  ObsPair c;
+  int64_t sg_b, sh_b, sn_b, so_b;
+  int B, H, first, np, nsplit;
+};
+
+// (min, max) over the wave, in every lane, with VALU lane moves.
+__device__ __forceinline__ void wave_minmax(float& mn, float& mx) {
+  static_for<0, 6>([&](auto I) {
+    mn = __builtin_fminf(mn, lane_xor_c<(1 << I)>(mn));
+    mx = __builtin_fmaxf(mx, lane_xor_c<(1 << I)>(mx));
+  });
+}
+
+// What step_scales reads, loaded by every thread before anything else: memory
+// returns in order, and behind the operand loads these would wait for all of
+// them (workgroup 0 for a second trip, in front of everyone else's step t + 1).
+struct StepIn {
+  float2 part[4];  // lanes past the last partial repeat it
+  float in[3], out[3], st[2];
+};
+
+__device__ __forceinline__ StepIn load_step_in(const OStep& p) {
+  StepIn v;
+  const int lane = threadIdx.x & 63;
 #pragma unroll
-      for (int q = 0; q < kMaxSplit; ++q)
+  for (int j = 0; j < 4; ++j) v.part[j] = p.part_in[min(lane + 64 * j, max(p.np, 1) - 1)];
+  const float* si = p.c.in.mode == GS_OBS_MIN_MAX ? p.c.in.stats : p.st;
+  const float* so = p.c.out.mode == GS_OBS_MIN_MAX ? p.c.out.stats : p.st;
 #pragma unroll
-        for (int g = 0; g < 3; ++g) v[q][g] = q < nsplit ? p[q * split_stride + g * H] : 0.0f;
+  for (int j = 0; j < 3; ++j) {
+    v.in[j] = si[j];
+    v.out[j] = so[j];
+  }
+  v.st[0] = p.st[0];
+  v.st[1] = p.st[1];
+  return v;
+}
+
+// observe() on statistics already in registers.
+__device__ __forceinline__ void observe_in(const Obs& o, float (&s)[3], float mn, float mx) {
+#pragma clang fp contract(off)
+  if (o.mode != GS_OBS_MIN_MAX) return;
+  s[0] = s[2] == 0.0f ? mn : kKeep * s[0] + kMix * mn;
+  s[1] = s[2] == 0.0f ? mx : kKeep * s[1] + kMix * mx;
+  s[2] = s[2] == 0.0f ? 1.0f : s[2];
 #pragma unroll
-      for (int g = 0; g < 3; ++g) {
-        float sum = v[0][g];
+  for (int j = 0; j < 3; ++j) o.stats[j] = s[j];
+}
+
+// Reduces the partials (each wave by itself: no barrier) and derives the scales
+// of step t: q_out for h_{t-1} (none at t = 0: h0 is not quantized) and q_in.
+// Workgroup 0 updates the statistics, the scale words and the trace.
+__device__ __forceinline__ void step_scales(const OStep& p, StepIn& v, DynQuant* qout, DynQuant* qin) {
+  float mn = v.part[0].x, mx = v.part[0].y;
 #pragma unroll
-        for (int q = 1; q < kMaxSplit; ++q)
-          if (q < nsplit) sum += v[q][g];
-        g3[g] = sum;
+  for (int j = 1; j < 4; ++j) {
+    mn = __builtin_fminf(mn, v.part[j].x);
+    mx = __builtin_fmaxf(mx, v.part[j].y);
+  }
+  for (int i = 256 + (threadIdx.x & 63); i < p.np; i += 64) {
+    const float2 w = p.part_in[i];
+    mn = __builtin_fminf(mn, w.x);
+    mx = __builtin_fmaxf(mx, w.y);
+  }
+  wave_minmax(mn, mx);
+  const bool writer = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
+  const bool din = is_dynamic(p.c.in), dout = is_dynamic(p.c.out);
+  float s_out = p.c.out.mode == GS_OBS_FROZEN ? p.c.out.scale : 1.0f;
+  float zp_out = p.c.out.mode == GS_OBS_FROZEN ? p.c.out.zp : 0.0f;
+  float s_in = p.c.in.mode == GS_OBS_FROZEN ? p.c.in.scale : 1.0f;
+  float zp_in = p.c.in.mode == GS_OBS_FROZEN ? p.c.in.zp : 0.0f;
+  if (!p.first) {
+    if (dout) {
+      scale_zp(p.c.out, mn, mx, &s_out, &zp_out);
+      if (writer) {
+        observe_in(p.c.out, v.out, mn, mx);
+        if (p.c.in.stats == p.c.out.stats) {  // one quantizer in both places
+#pragma unroll
+          for (int j = 0; j < 3; ++j) v.in[j] = v.out[j];
+        }
       }
     }
-    const float* gr = gi_t + (int64_t)b * sg_b + k;
-    const float v = gru_update(gr[0], gr[H], gr[2 * H], g3[0], g3[1], g3[2], hprev[(int64_t)b * shp_b + k]);
-    out_t[(int64_t)b * so_b + k] = v;
+    if (writer && p.trace != nullptr) {
+      p.trace[0] = din ? v.st[0] : s_in;  // what step t - 1 used
+      p.trace[1] = din ? v.st[1] : zp_in;
+      p.trace[2] = s_out;
+      p.trace[3] = zp_out;
+    }
+    if (p.c.out.mode != GS_OBS_OFF) {
+      mn = fq(mn, s_out, zp_out, p.c.out.qmin, p.c.out.qmax);
+      mx = fq(mx, s_out, zp_out, p.c.out.qmin, p.c.out.qmax);
+    }
+  }
+  if (din) {
+    scale_zp(p.c.in, mn, mx, &s_in, &zp_in);
+    if (writer) {
+      observe_in(p.c.in, v.in, mn, mx);
+      p.st[0] = s_in;
+      p.st[1] = zp_in;
+    }
+  }
+  *qout = dyn_quant(p.c.out, s_out, zp_out);
+  if (p.first) qout->on = qout->fast = 0;
+  *qin = dyn_quant(p.c.in, s_in, zp_in);
+  // q_in repeats q_out: the levels it sees are its own (same_quant, gs_host.h)
+  if (qout->fast && qin->fast && s_in == s_out && p.c.in.qmin == p.c.out.qmin && p.c.in.qmax == p.c.out.qmax)
+    qin->on = qin->fast = 0;
+}
+
+// (min, max) over the workgroup into *dst; red holds two floats per wave.
+template <int NW>
+__device__ __forceinline__ void wg_minmax(float mn, float mx, float2* red, float2* dst) {
+  wave_minmax(mn, mx);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = float2{mn, mx};
+  lds_barrier();  // (not the stores of the step: their acknowledgements would be waited for)
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < NW; ++w) {
+      mn = __builtin_fminf(mn, red[w].x);
+      mx = __builtin_fmaxf(mx, red[w].y);
+    }
+    *dst = float2{mn, mx};
+  }
+}
+
+// A workgroup of 8 waves owns 16 RT batch rows x 16 units (three gates); wave q
+// runs K split q of the product (gemm.hip's NT kernel with K split in up to 8:
+// 16x16x4 MFMAs over 32-k slices in its k order, the splits added in order, so
+// gh is that GEMM's bit for bit) from an LDS staging of its own, without a
+// barrier, NS slices in flight, quantizing the state's rows as it stages them; the
+// splits meet in LDS once. Bound: one launch of about 3.3 us, two dependent trips
+// to memory (partials, then operands to use) and the product. us a step at B = 32,
+// H = 512: GEMM 7.0, gates 3.8 and quantizers 3.8 as three launches, 13.8 together
+// -> 8.0; B = 256, H = 512 23.0 -> 11.2; B = 32, H = 1024 18.7 -> 11.2; H = 64 12.7 -> 5.9.
+constexpr int kObsRS = 40;  // LDS row stride of a 32-k slice (gemm.hip)
+
+template <int RT, bool RAG, int NS>
+__global__ __launch_bounds__(512) void observe_step_kernel(OStep p) {
+  extern __shared__ __attribute__((aligned(16))) float olds[];
+  __shared__ float2 red2[8];
+  constexpr int NR = 16 * RT + 48;  // staged rows: the state's, then 16 units of each gate
+  constexpr int NL = NR / 8;        // 16-byte loads a lane and slice (8 lanes a row)
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int H = p.H;
+  const int u0 = 16 * blockIdx.x, row0 = 16 * RT * blockIdx.y;
+  float* mine = olds + wave * NR * kObsRS;
+  StepIn in = load_step_in(p);
+  __builtin_amdgcn_sched_barrier(0);
+
+  const int kper = ((H + p.nsplit - 1) / p.nsplit + 31) / 32 * 32;
+  const int kbeg = wave * kper, kend = wave < p.nsplit ? min(H, kbeg + kper) : 0;
+  const int r8 = lane >> 3, k4 = 4 * (lane & 7);
+  const float* src[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int r = 8 * i + r8;
+    src[i] = i < 2 * RT ? p.hprev + (int64_t)min(row0 + r, p.B - 1) * p.sh_b
+                        : p.w + ((int64_t)((r - 16 * RT) >> 4) * H + min(u0 + (r & 15), H - 1)) * H;
+  }
+  // elements k .. k + 3 of each row; what lies past the end is zeroed at staging
+  // (RAG: the lane across a row's end loads its last four)
+  f4 x[NS][NL];  // slices in flight
+  auto load = [&](int k0, f4 (&v)[NL]) __attribute__((always_inline)) {
+    const int k = k0 + k4;
+    if (RAG && H < 4) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[i][e] = src[i][k + e < H ? k + e : 0];
+      return;
+    }
+    const int kk = RAG ? min(k, H - 4) : k < H ? k : 0;
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+    for (int i = 0; i < NL; ++i) v[i] = *reinterpret_cast<const f4u*>(src[i] + kk);
+  };
+  static_for<0, NS>([&](auto I) { load(kbeg + 32 * I, x[I]); });
+
+  // the epilogue's element: row 16 (wave / 4) + 4 (lane / 16) + wave % 4, unit lane % 16
+  const int er = row0 + 16 * (wave >> 2) + 4 * (lane >> 4) + (wave & 3), eu = u0 + (lane & 15);
+  const bool mineq = wave < 4 * RT;
+  const bool live = mineq && er < p.B && eu < H;
+  const int64_t erc = min(er, p.B - 1);
+  const int euc = min(eu, H - 1);
+  float gin[3], bb[3];
+#pragma unroll
+  for (int g = 0; g < 3; ++g) {
+    gin[g] = p.gi[erc * p.sg_b + g * H + euc];
+    bb[g] = p.bh[g * H + euc];
+  }
+  const float hraw = p.hprev[erc * p.sh_b + euc];
+
+  DynQuant qout, qin;
+  step_scales(p, in, &qout, &qin);
+
+  // one division-free quantizer for the state (the common case): applied as the rows are staged
+  const bool one_quant = (qout.fast && !qin.on) || (qin.fast && !qout.on);
+  const Quant q1 = qout.on ? qout.q : qin.q;
+
+  f4 acc[RT][3];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int g = 0; g < 3; ++g) acc[i][g] = f4{0.f, 0.f, 0.f, 0.f};
+  const int r16 = lane & 15, kq = lane >> 4;
+  auto slice = [&](int k0, f4 (&v)[NL]) __attribute__((always_inline)) {
+    const int k = k0 + k4;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      f4 y = v[i];
+      if (RAG && k0 + 32 > H && H >= 4) {  // (uniform)
+        const int s = k - (H - 4);  // 1 .. 3: the lane across the end, its last four loaded
+        if (s == 1) y = f4{y[1], y[2], y[3], 0.f};
+        if (s == 2) y = f4{y[2], y[3], 0.f, 0.f};
+        if (s == 3) y = f4{y[3], 0.f, 0.f, 0.f};
+      }
+      if (i < 2 * RT && one_quant) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = quant_level(y[e], q1) * q1.scale;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = k + (RAG ? e : 0) < kend ? y[e] : 0.0f;
+      *reinterpret_cast<f4*>(mine + (8 * i + r8) * kObsRS + k4) = y;
+    }
+    if (!one_quant) {  // affine, off or different quantizers: in place, a loop to keep the code short
+#pragma unroll 1
+      for (int i = 0; i < 8 * RT; ++i) {
+        float* h = mine + (8 * (i >> 2) + r8) * kObsRS + k4 + (i & 3);
+        *h = k + (RAG ? i & 3 : 0) < kend ? qin(qout(*h)) : 0.0f;
+      }
+    }
+    // (a wave's LDS accesses complete in order: no barrier within the wave's own staging)
+    f4 a[RT][2], b[3][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+        a[i][h] = *reinterpret_cast<const f4*>(mine + (16 * i + r16) * kObsRS + 4 * kq + 16 * h);
+#pragma unroll
+      for (int g = 0; g < 3; ++g)
+        b[g][h] = *reinterpret_cast<const f4*>(mine + (16 * (RT + g) + r16) * kObsRS + 4 * kq + 16 * h);
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int g = 0; g < 3; ++g)
+          acc[i][g] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][s >> 2][s & 3], b[g][s >> 2][s & 3], acc[i][g], 0, 0, 0);
+  };
+  for (int k0 = kbeg; k0 < kend; k0 += 32 * NS) {
+    const bool more = k0 + 32 * NS < kend;
+    static_for<0, NS>([&](auto I) {
+      if (I < 2 || k0 + 32 * I < kend) slice(k0 + 32 * I, x[I]);  // (a slice past kend adds zeros)
+      if (more) load(k0 + 32 * (NS + I), x[I]);
+    });
+  }
+
+  float* red = mine;  // [RT * 3][v][lane] in the wave's own staging
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int g = 0; g < 3; ++g)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[((i * 3 + g) * 4 + v) * 64 + lane] = acc[i][g][v];
+  lds_barrier();
+  float mn = __builtin_inff(), mx = -__builtin_inff();
+  if (mineq) {
+    float g3[3];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      const float* q = olds + (((wave >> 2) * 3 + g) * 4 + (wave & 3)) * 64 + lane;
+      float sum = q[0] + bb[g];
+#pragma unroll
+      for (int w = 1; w < kMaxSplit; ++w)
+        if (w < p.nsplit) sum += q[w * NR * kObsRS];
+      g3[g] = sum;
+    }
+    if (live) {
+      const float h = qout(hraw);
+      if (p.out_prev != nullptr) p.out_prev[er * p.so_b + eu] = h;
+      const float v = gru_update(gin[0], gin[1], gin[2], g3[0], g3[1], g3[2], h);
+      p.hnext[er * p.sn_b + eu] = v;
+      mn = mx = v;
+      if (!(v == v)) {  // a NaN takes no part, as in the other reductions
+        mn = __builtin_inff();
+        mx = -__builtin_inff();
+      }
+    }
+  }
+  wg_minmax<8>(mn, mx, red2, p.part_out + (int64_t)blockIdx.y * gridDim.x + blockIdx.x);
+}
+
+// The diagonal kind's step: every element is its own, so the pre-quant h_t goes
+// to out[t] and is quantized in place a launch later. As two launches a step
+// (gates 3.8 us, quantizers 3.8) it took 6.4 us at B = 32, H = 512, here 4.0.
+__global__ __launch_bounds__(kRedThreads) void observe_diag_kernel(OStep p) {
+  __shared__ float2 red2[kRedThreads / 64];
+  StepIn in = load_step_in(p);
+  DynQuant qout, qin;
+  step_scales(p, in, &qout, &qin);
+  const int H = p.H;
+  float mn = __builtin_inff(), mx = -__builtin_inff();
+  const int64_t n = (int64_t)p.B * H;
+  for (int64_t e = blockIdx.x * (int64_t)kRedThreads + threadIdx.x; e < n; e += (int64_t)gridDim.x * kRedThreads) {
+    const int b = (int)(e / H), k = (int)(e - (int64_t)b * H);
+    const float h = qout(p.hprev[(int64_t)b * p.sh_b + k]);
+    if (p.out_prev != nullptr && qout.on) p.out_prev[(int64_t)b * p.so_b + k] = h;
+    const float hq = qin(h);
+    float g3[3];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+#pragma clang fp contract(off)
+      g3[g] = p.w[g * H + k] * hq + p.bh[g * H + k];
+    }
+    const float* gr = p.gi + (int64_t)b * p.sg_b + k;
+    const float v = gru_update(gr[0], gr[H], gr[2 * H], g3[0], g3[1], g3[2], h);
+    p.hnext[(int64_t)b * p.sn_b + k] = v;
     mn = __builtin_fminf(mn, v);
     mx = __builtin_fmaxf(mx, v);
   }
-  block_minmax(mn, mx, part + blockIdx.x);
+  wg_minmax<kRedThreads / 64>(mn, mx, red2, p.part_out + blockIdx.x);
+}
+
+// One (min, max) from n: a step of very many workgroups, whose partials every
+// workgroup of the next would read.
+__global__ __launch_bounds__(1024) void reduce_partials_kernel(const float2* part, int n, float2* dst) {
+  __shared__ float2 red2[16];
+  float mn = __builtin_inff(), mx = -__builtin_inff();
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    mn = __builtin_fminf(mn, part[i].x);
+    mx = __builtin_fmaxf(mx, part[i].y);
+  }
+  wg_minmax<16>(mn, mx, red2, dst);
 }
 
 int validate_observer(const gs_observer& o, const char* name, const char* who) {
@@ -300,13 +628,16 @@ unsigned parts_for(int64_t n) { return (unsigned)std::min<int64_t>((n + kRedThre
 dim3 grid1d(int64_t n) { return dim3((unsigned)std::min<int64_t>((n + 255) / 256, 8192)); }
 
 // Scratch of gs_observe_scan, each region 256-byte aligned:
-// scales [4] | partials [kMaxParts] | hq [B, H] | gh [split][B, 3H] |
-// map [3H, H] (Monarch, butterfly) | map construction scratch.
+// scales [4] | partials of two steps | pre-quant h of two steps [2][B, H] (not
+// the diagonal kind) | map [3H, H] (Monarch, butterfly, circulant) | map
+// construction scratch.
 struct OPlan {
   bool gemm, own_map;
   int split;
-  int64_t st, part, hq, gh, map, map_tmp;
-  int64_t total() const { return st + part + hq + gh + map + map_tmp; }
+  int rt;       // 16-row tiles a workgroup (1 or 2)
+  int64_t nwg;  // workgroups, and partials, of a step
+  int64_t st, part, hpre, map, map_tmp;
+  int64_t total() const { return st + 2 * part + 2 * hpre + map + map_tmp; }
 };
 
 gs_map_args map_view(const gs_observe_args* a) {
@@ -352,13 +683,15 @@ int plan_observe(const gs_observe_args* a, OPlan* p, const char* who) {
     return set_error(GS_ERR_INVALID, "%s: B * 3H = %lld is too large", who, (long long)(B * 3 * H));
   p->gemm = a->kind != GS_KIND_DIAGONAL;
   p->own_map = a->kind == GS_KIND_MONARCH || a->kind == GS_KIND_BUTTERFLY || a->kind == GS_KIND_CIRCULANT;
-  // gh has only B rows: split K in up to 8 parts of >= 64 terms so that the
-  // product spreads over a few hundred workgroups (the gates kernel sums them).
+  // gh has only B rows: split K in up to 8 parts of >= 64 terms, one wave each
   p->split = p->gemm ? (int)std::max<int64_t>(1, std::min<int64_t>(kMaxSplit, H / 64)) : 1;
+  // 32 rows a workgroup (Wh read half as often) once 16 give every CU one
+  const int64_t nut = (H + 15) / 16;
+  p->rt = ((B + 15) / 16) * nut > 256 ? 2 : 1;
+  p->nwg = p->gemm ? ((B + 16 * p->rt - 1) / (16 * p->rt)) * nut : parts_for(B * H);
   p->st = 256;
-  p->part = align256((int64_t)kMaxParts * 8);
-  p->hq = align256(B * H * 4);
-  p->gh = p->gemm ? align256((int64_t)p->split * B * 3 * H * 4) : 0;
+  p->part = align256(std::max<int64_t>(p->nwg, kMaxParts) * 8);
+  p->hpre = p->gemm ? align256(B * H * 4) : 0;
   p->map = p->own_map ? align256(3 * H * H * 4) : 0;
   p->map_tmp = p->own_map ? hidden_map_scratch(&m) : 0;
   return GS_OK;
@@ -393,15 +726,16 @@ extern "C" int gs_observe_scan(const gs_observe_args* a, hipStream_t stream) {
     return r;
   };
   float* st = reinterpret_cast<float*>(take(p.st));
-  float2* part = reinterpret_cast<float2*>(take(p.part));
-  float* hq = reinterpret_cast<float*>(take(p.hq));
-  float* gh = reinterpret_cast<float*>(take(p.gh));
+  float2* part[2];
+  for (float2*& q : part) q = reinterpret_cast<float2*>(take(p.part));
+  float* hpre[2];
+  for (float*& q : hpre) q = reinterpret_cast<float*>(take(p.hpre));
   float* map = reinterpret_cast<float*>(take(p.map));
   void* map_tmp = take(p.map_tmp);
 
   const int T = (int)a->T, B = (int)a->B, H = (int)a->H;
   const ObsPair c{to_obs(a->q_in), to_obs(a->q_out)};
-  const bool in_on = a->q_in.mode != GS_OBS_OFF, out_on = a->q_out.mode != GS_OBS_OFF;
+  const bool out_on = a->q_out.mode != GS_OBS_OFF;
   const int64_t BH = (int64_t)B * H;
 
   const float* W = a->w;
@@ -414,53 +748,65 @@ extern "C" int gs_observe_scan(const gs_observe_args* a, hipStream_t stream) {
     if (rc) return rc;
     W = map;
   }
-  const unsigned np = parts_for(BH);
+  const bool any_dyn = is_dynamic(c.in) || is_dynamic(c.out);
+  int np = 0;
   if (is_dynamic(c.in)) {
-    hipLaunchKernelGGL(minmax_partials, dim3(np), dim3(kRedThreads), 0, stream, a->h0, (int64_t)B, H, a->sh0_b, part);
-    GS_CHECK_HIP(hipGetLastError());
-  }
-  if (in_on) {
-    hipLaunchKernelGGL(quant_step, grid1d(BH), dim3(kRedThreads), 0, stream, part, is_dynamic(c.in) ? (int)np : 0, c,
-                       st, a->trace, 0, T, 0, a->h0, a->sh0_b, nullptr, (int64_t)0, hq, (int64_t)B, H, 0);
+    np = (int)parts_for(BH);
+    hipLaunchKernelGGL(minmax_partials, dim3((unsigned)np), dim3(kRedThreads), 0, stream, a->h0, (int64_t)B, H,
+                       a->sh0_b, part[1]);
     GS_CHECK_HIP(hipGetLastError());
   }
 
+  const unsigned nut = (unsigned)((H + 15) / 16);
+  const dim3 grid = p.gemm ? dim3(nut, (unsigned)(p.nwg / nut)) : dim3((unsigned)p.nwg);
+  const bool rag = H % 4 != 0;
+  void (*fn)(OStep) = !p.gemm ? observe_diag_kernel
+                      : p.rt == 2 ? (rag ? observe_step_kernel<2, true, 2> : observe_step_kernel<2, false, 2>)
+                      : H > 64 * p.split ? (rag ? observe_step_kernel<1, true, 4> : observe_step_kernel<1, false, 4>)
+                                         : (rag ? observe_step_kernel<1, true, 2> : observe_step_kernel<1, false, 2>);
+  const int lds = p.gemm ? 8 * (16 * p.rt + 48) * kObsRS * 4 : 0;
+  if (lds > 65536) GS_CHECK_HIP(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  OStep s;
+  s.w = W;
+  s.bh = a->bh;
+  s.st = st;
+  s.c = c;
+  s.sg_b = a->sg_b;
+  s.so_b = a->so_b;
+  s.B = B;
+  s.H = H;
+  s.nsplit = p.split;
   for (int t = 0; t < T; ++t) {
-    const float* hprev = t == 0 ? a->h0 : a->out + (int64_t)(t - 1) * a->so_t;
-    const int64_t shp = t == 0 ? a->sh0_b : a->so_b;
-    const float* hm = in_on ? hq : hprev;  // the matmul-side h
-    const int64_t shm = in_on ? H : shp;
+    s.gi = a->gi + (int64_t)t * a->sg_t;
     float* out_t = a->out + (int64_t)t * a->so_t;
-    if (p.gemm) {
-      GemmArgs g;
-      g.a = hm;
-      g.lda = shm;
-      g.b = W;  // B(k, n) = W[n][k]
-      g.ldb = H;
-      g.c = gh;
-      g.ldc = 3 * H;
-      g.split_stride = (int64_t)B * 3 * H;
-      g.bias = a->bh;
-      g.M = B;
-      g.N = 3 * H;
-      g.K = H;
-      g.ksplit = p.split;
-      g.layout = kGemmNT;
-      rc = gemm_f32(g, stream, who);
-      if (rc) return rc;
+    s.out_prev = t == 0 ? nullptr : out_t - a->so_t;
+    s.hprev = t == 0 ? a->h0 : p.gemm ? hpre[(t - 1) & 1] : s.out_prev;
+    s.sh_b = t == 0 ? a->sh0_b : p.gemm ? H : a->so_b;
+    s.hnext = p.gemm ? hpre[t & 1] : out_t;
+    s.sn_b = p.gemm ? H : a->so_b;
+    s.part_in = part[(t + 1) & 1];
+    s.part_out = part[t & 1];
+    s.trace = t > 0 && a->trace != nullptr ? a->trace + (int64_t)(t - 1) * 4 : nullptr;
+    s.first = t == 0;
+    s.np = np;
+    hipLaunchKernelGGL(fn, grid, dim3(p.gemm ? 512 : kRedThreads), (size_t)lds, stream, s);
+    GS_CHECK_HIP(hipGetLastError());
+    np = any_dyn ? (int)p.nwg : 0;
+    if (np > 2 * kMaxParts) {
+      // the workgroups of step t have read part[(t + 1) & 1]
+      hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(1024), 0, stream, part[t & 1], np, part[(t + 1) & 1]);
+      GS_CHECK_HIP(hipGetLastError());
+      std::swap(part[0], part[1]);  // its one pair is the next step's input
+      np = 1;
     }
-    hipLaunchKernelGGL(gates_step, dim3(np), dim3(kRedThreads), 0, stream, a->gi + (int64_t)t * a->sg_t, a->sg_b,
-                       gh, p.split, (int64_t)B * 3 * H, p.gemm ? nullptr : a->w, a->bh, hm, shm, hprev, shp, out_t,
-                       a->so_b, B, H, part);
-    GS_CHECK_HIP(hipGetLastError());
-    // q_out's pass runs every step: it also writes the trace
-    const bool any_dyn = is_dynamic(c.in) || is_dynamic(c.out);
-    float* hq_next = (in_on && t + 1 < T) ? hq : nullptr;
-    hipLaunchKernelGGL(quant_step, grid1d(BH), dim3(kRedThreads), 0, stream, part, any_dyn ? (int)np : 0, c, st,
-                       a->trace, t, T, 1, out_t, a->so_b, out_on ? out_t : nullptr, a->so_b, hq_next, (int64_t)B, H,
-                       out_on ? 1 : 0);
-    GS_CHECK_HIP(hipGetLastError());
   }
+  // out[T-1] and the last trace entry
+  float* out_t = a->out + (int64_t)(T - 1) * a->so_t;
+  const float* x = p.gemm ? hpre[(T - 1) & 1] : out_t;
+  hipLaunchKernelGGL(quant_step, grid1d(BH), dim3(kRedThreads), 0, stream, part[(T - 1) & 1], np, c, st, a->trace,
+                     T - 1, T, 1, x, p.gemm ? (int64_t)H : a->so_b, p.gemm || out_on ? out_t : nullptr, a->so_b,
+                     nullptr, (int64_t)B, H, out_on ? 1 : 0);
+  GS_CHECK_HIP(hipGetLastError());
   return GS_OK;
 }
 

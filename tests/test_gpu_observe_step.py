@@ -1,0 +1,67 @@
+"""The observer scan's one launch per step (observe.hip) at the edges of its
+tiles: 16 units, 16 or 32 rows, K splits of 32-k slices, row ends of every
+length, more partials than a workgroup reads, one quantizer in both places.
+Checked step by step from the kernel's own previous output, as in
+test_gpu_observe.py."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import gru_qat_amd as G
+from oracle import gru_oracle as O
+from test_gpu_observe import _cfg, _codes_match, _quant, _run, _teacher_forced
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [(3, 2, 1), (3, 2, 3), (3, 17, 6), (3, 15, 33), (2, 33, 127), (2, 16, 130), (2, 3, 517),
+                                   (2, 280, 257),     # 32 rows a workgroup
+                                   (2, 2200, 256)])   # 1104 partials: reduced by a launch of their own
+@pytest.mark.parametrize("mode,symmetric", [("min_max", True), ("dynamic", False)])
+def test_observe_step_edges(dev, shape, mode, symmetric):
+    cfg = _cfg(1, shape)
+    q_in, q_out = _quant(mode, symmetric).to(dev), _quant(mode, symmetric).to(dev)
+    out, trace = _run(cfg, dev, q_in, q_out)
+    out, trace = out.cpu(), trace.cpu()
+    st_in, st_out = O.ObserverState(mode, symmetric=symmetric), O.ObserverState(mode, symmetric=symmetric)
+    pre, sc = _teacher_forced(cfg, out, st_in, st_out)
+    assert torch.equal(trace[:, :2], sc[:, :2])
+    assert torch.allclose(trace[:, 2], sc[:, 2], rtol=1e-5, atol=0)
+    for t in range(shape[0]):
+        _codes_match(out[t], pre[t], float(trace[t, 2]), float(trace[t, 3]), q_out.qmin, q_out.qmax)
+    if mode == "min_max":
+        assert torch.equal(q_in.observer_stats.cpu()[:2], torch.stack([st_in.running_min, st_in.running_max]))
+
+
+@pytest.mark.parametrize("idx,shape", [(1, (4, 5, 96)), (0, (4, 5, 96))])
+def test_observe_one_quantizer_in_both_places(dev, idx, shape):
+    cfg = _cfg(idx, shape)
+    q = _quant("min_max", True).to(dev)
+    out, _ = _run(cfg, dev, q, q)
+    st = O.ObserverState("min_max")
+    _teacher_forced(cfg, out.cpu(), st, st)
+    assert torch.allclose(q.observer_stats.cpu()[:2], torch.stack([st.running_min, st.running_max]), rtol=1e-5)
+
+
+@pytest.mark.parametrize("idx", [0, 1])
+@pytest.mark.parametrize("which", ["in", "out"])
+def test_observe_one_side_off(dev, idx, which):
+    cfg = _cfg(idx, (4, 19, 70))
+    q = _quant("min_max", True).to(dev)
+    out, trace = _run(cfg, dev, q if which == "in" else None, q if which == "out" else None)
+    out = out.cpu()
+    c = {k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in cfg.items()}
+    gh_fn, st = O.gh_fn_for(c), O.ObserverState("min_max")
+    for t in range(out.shape[0]):
+        h = c["h0"] if t == 0 else out[t - 1]
+        hq = O.observer_forward(st, h)[0] if which == "in" else h
+        pre = O.gru_step(c["gi"][t], h, gh_fn(hq))
+        if which == "in":
+            assert (out[t] - pre).abs().max() <= 1e-5
+        else:
+            s = O.observer_forward(st, pre)[1][0]
+            assert abs(float(trace[t, 2]) - s) <= 1e-5 * s
+            _codes_match(out[t], pre, float(trace[t, 2]), 0.0, -127, 127)
+    assert torch.allclose(q.observer_stats.cpu()[:2], torch.stack([st.running_min, st.running_max]), rtol=1e-5)
