@@ -59,7 +59,6 @@ namespace {
 
 constexpr int kGemmThreads = 256;
 constexpr int kSmallT = 64, kBigT = 128;
-constexpr int kSpread = 64;  // from so many tiles on, each XCD takes a run of them
 constexpr int kSplitK = 32;  // K splits start at multiples of this: whole slices of either tile
 
 // How an operand's tile is loaded: 16 bytes or one float per buffer load, or
@@ -176,8 +175,13 @@ __device__ __forceinline__ void interleave() {
 }
 
 // Q: fake-quantizes A (NT) or B (TN) on its way to LDS.
+// Four workgroups of NT's small tiles fit a CU, which short products, bound by
+// their stores, are the faster for (M = 16384, N = 1536, K = 64: 60 -> 53 us);
+// NN and TN lose more to the registers (their backward 112 -> 116 us).
 template <int LAYOUT, int T, int LOAD, bool Q>
-__global__ __launch_bounds__(kGemmThreads, T == kBigT || LOAD == kLoadFar ? 2 : 3) void gemm_kernel(GemmArgs g) {
+__global__ __launch_bounds__(kGemmThreads, T == kBigT || LOAD == kLoadFar                ? 2
+                                           : LAYOUT == kGemmNT && LOAD == kLoadVec ? 4
+                                                                                   : 3) void gemm_kernel(GemmArgs g) {
   constexpr bool A_KC = LAYOUT != kGemmTN, B_KC = LAYOUT == kGemmNT, TN = LAYOUT == kGemmTN;
   constexpr bool QA = Q && LAYOUT == kGemmNT, QB = Q && LAYOUT == kGemmTN;
   constexpr int RS = T + (LAYOUT == kGemmNN ? 4 : 16);
@@ -186,14 +190,12 @@ __global__ __launch_bounds__(kGemmThreads, T == kBigT || LOAD == kLoadFar ? 2 : 
   constexpr int BK = LA::BK, MT = T / 32, KH = BK / 16;
   __shared__ __attribute__((aligned(16))) float As[2][LA::kStage];
   __shared__ __attribute__((aligned(16))) float Bs[2][LB::kStage];
-  // this workgroup's tile: each XCD (workgroup mod 8) takes a run of tiles, in
-  // patches of 1024 rows, whose operands its L2 then holds (the grid is a
-  // multiple of 8 workgroups wide then; products of few tiles are not spread)
+  // this workgroup's tile: patches of 1024 rows; of big tiles, each XCD
+  // (workgroup mod 8) takes a run, whose operands its L2 then holds
   const int mt = (g.M + T - 1) / T, nt = (g.N + T - 1) / T, total = mt * nt;
-  const int per = (total + 7) / 8;
-  const int wg = blockIdx.y * gridDim.x + blockIdx.x;
-  const int tile = total < kSpread ? wg : (wg & 7) * per + (wg >> 3);
-  if ((total >= kSpread && (wg >> 3) >= per) || tile >= total) return;  // uniform
+  const int wg = blockIdx.y * gridDim.x + blockIdx.x, per = (total + 7) / 8;
+  const int tile = T == kBigT ? (wg & 7) * per + (wg >> 3) : wg;
+  if ((T == kBigT && (wg >> 3) >= per) || tile >= total) return;  // uniform
   constexpr int kPatch = 1024 / T;
   const int patch = tile / (kPatch * nt), in_patch = tile - patch * kPatch * nt;
   const int pm = min(kPatch, mt - patch * kPatch);
@@ -236,15 +238,7 @@ __global__ __launch_bounds__(kGemmThreads, T == kBigT || LOAD == kLoadFar ? 2 : 
   };
   constexpr std::integral_constant<int, 0> I0{};
   constexpr std::integral_constant<int, 1> I1{};
-  put(0, I0);
-  put(1, I1);
-  lds_barrier();
-  read(I0);
-  // slice s + 2 is staged where slice s was: every wave read that one before
-  // the barrier that ended slice s - 1
-  auto slice = [&](int s, auto I, auto J) __attribute__((always_inline)) {
-    read(J);
-    put(s + 2, I);
+  auto products = [&](auto I) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < 4 * KH; ++e)
 #pragma unroll
@@ -253,15 +247,30 @@ __global__ __launch_bounds__(kGemmThreads, T == kBigT || LOAD == kLoadFar ? 2 : 
         for (int tj = 0; tj < MT; ++tj)
           acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(oa[I][ti][e >> 2][e & 3], ob[I][tj][e >> 2][e & 3],
                                                              acc[ti][tj], 0, 0, 0);
+  };
+  put(0, I0);
+  if (n > 1) put(1, I1);
+  lds_barrier();
+  read(I0);
+  lds_barrier();  // slice 0 is read: its half of the LDS takes slice 2
+  // slice s + 2 is staged where slice s was: every wave read that one before
+  // the barrier that ended slice s - 1
+  auto slice = [&](int s, auto I, auto J) __attribute__((always_inline)) {
+    read(J);
+    put(s + 2, I);
+    products(I);
     interleave<4 * KH * MT * MT, MT * KH * ((A_KC ? 1 : 4) + (B_KC ? 1 : 4)), LA::NV + LB::NV>();
     lds_barrier();
   };
-  lds_barrier();  // slice 0 is read: its half of the LDS takes slice 2
-  // pairs of slices (one past the last adds zeros), so that the loop has one exit
-  for (int s = 0; s < n; s += 2) {
+  int s = 0;
+  for (; s + 2 < n; s += 2) {  // in pairs, so that the loop has one exit
     slice(s, I0, I1);
     slice(s + 1, I1, I0);
   }
+  // the last one or two: nothing further to stage
+  if (s + 1 < n) read(I1);
+  if (s < n) products(I0);
+  if (s + 1 < n) products(I1);
 
   float* c = g.c + (int64_t)z * g.c_bs + (int64_t)split * g.split_stride;
   const float* biasp = g.bias ? g.bias + (int64_t)z * g.bias_bs : nullptr;
@@ -542,8 +551,8 @@ int gemm_f32(const GemmArgs& g, hipStream_t stream, const char* who) {
     return set_error(GS_ERR_INVALID, "%s: GEMM layout %d quantizes no such operand", who, g.layout);
   GemmFn fn = table[g.layout][big ? 3 + load : load][quant ? 1 : 0];
   int64_t tiles = tile_count(g.M, g.N, big ? kBigT : kSmallT);
-  if (tiles >= kSpread) tiles = 8 * ((tiles + 7) / 8);
-  const int64_t gx = std::min<int64_t>(tiles, 1 << 20);  // a multiple of 8, as tiles is from kSpread on
+  if (big) tiles = 8 * ((tiles + 7) / 8);
+  const int64_t gx = std::min<int64_t>(tiles, 1 << 20);  // for big tiles a multiple of 8
   if (tiles > INT32_MAX || (tiles + gx - 1) / gx > 65535)
     return set_error(GS_ERR_INVALID, "%s: GEMM of too many tiles (M=%d, N=%d)", who, g.M, g.N);
   const dim3 grid((unsigned)gx, (unsigned)((tiles + gx - 1) / gx), (unsigned)(g.batch * g.ksplit));
