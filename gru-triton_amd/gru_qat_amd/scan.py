@@ -8,18 +8,19 @@ Entry points keep the reference signatures
   persistent kernels ``gs_dense_fwd`` / ``gs_dense_bwd`` (one launch, Wh resident
   in registers, the state exchanged between workgroups every step, fp32 MFMA);
 * ``gru_scan(...)`` (scan.py:1607-1627) and ``GRUScanFunction`` (scan.py:1556-1604),
-  same contract, on the barrier-free batch-tiled kernels ``gs_dense_fwd_tiled`` /
-  ``gs_dense_bwd_tiled`` (one workgroup per tile of batch rows, Wh read from
+  same contract, on the barrier-free kernels ``gs_dense_fwd_tiled`` /
+  ``gs_dense_bwd_tiled`` (one launch per step over the whole batch, or, for
+  H <= 128 and short work, one workgroup per tile of batch rows; Wh read from
   memory every step, no co-residency requirement), as the reference's
   ``gru_scan`` runs its non-persistent kernels (scan.py:755-913, :916-1352);
 * the forward-only launchers ``gru_scan_forward_persistent`` (scan.py:213-293,
-  persistent) and ``gru_scan_forward`` (scan.py:1688-1765, batch-tiled), and the
+  persistent) and ``gru_scan_forward`` (scan.py:1688-1765, barrier-free), and the
   backward launchers ``gru_scan_backward_persistent`` (scan.py:646-752) and
-  ``gru_scan_backward_triton`` (scan.py:1355-1447, batch-tiled).
+  ``gru_scan_backward_triton`` (scan.py:1355-1447, barrier-free).
 
 Both kernel families compute the same products in the same order, so their
 outputs are bit-identical up to H = 1024; above that the persistent entry
-points run the batch-tiled kernels too (up to H = 8192).
+points run the barrier-free kernels too (up to H = 8192).
 
 ``Wh_cat`` is ``[3H, H]`` with rows ordered r, z, n and ``gh = hq @ Wh_cat.T +
 bh_cat``. ``h_in_quant`` / ``h_out_quant`` are optional frozen per-tensor

@@ -133,18 +133,20 @@ typedef struct gs_args {
 
 /* Dense forward. H <= 1024: the persistent kernel (Wh resident in registers, the state
  * exchanged between workgroups every step, a workspace of gs_workspace_bytes() bytes).
- * 1024 < H <= 8192: the batch-tiled kernel of gs_dense_fwd_tiled (same results,
- * no workspace: gs_workspace_bytes() returns 0). */
+ * Large batches, whose row blocks the persistent groups would take many in turn, run one
+ * launch per step instead (the workspace stays required). 1024 < H <= 8192: the kernels of
+ * gs_dense_fwd_tiled (same results, no workspace: gs_workspace_bytes() returns 0). */
 int gs_dense_fwd(const gs_args* args, hipStream_t stream);
 
 /* Barrier-free dense forward (reference gru_scan_fwd_kernel, scan.py:755-913, launched
- * by gru_scan_forward, scan.py:1688-1765): a 1-D grid over tiles of up to 4 batch rows,
- * each workgroup running every step of its rows and reading Wh from memory each step,
- * so no workgroup waits for another: no co-residency requirement, no workspace
- * (workspace and fault_mirror are ignored), no poll bound. 1 <= H <= 8192.
- * Same products and gate arithmetic as gs_dense_fwd, so at H <= 1024 the two return
- * bit-identical outputs; gs_dense_fwd is the faster of the two there (each step here
- * streams all 3 H^2 weights through one CU). gh_save as for gs_dense_fwd. */
+ * by gru_scan_forward, scan.py:1688-1765): one launch per step over the whole batch from
+ * H = 129 on; below, and where a step launch does not apply (out overlapping an input,
+ * row strides past 2^22 floats, few short steps), one launch over tiles of up to 4 batch
+ * rows, each workgroup running every step of its rows. Either way no workgroup waits for
+ * another: no co-residency requirement, no workspace (workspace and fault_mirror are
+ * ignored), no poll bound. 1 <= H <= 8192. Same products and gate arithmetic as
+ * gs_dense_fwd, so at H <= 1024 the two return bit-identical outputs; gs_dense_fwd is the
+ * faster of the two there for batches up to 32. gh_save as for gs_dense_fwd. */
 int gs_dense_fwd_tiled(const gs_args* args, hipStream_t stream);
 
 /* Dense forward with Wh also given as per-row int8 codes: w_codes [3H, H] int8
@@ -275,15 +277,15 @@ int gs_diagonal_bwd(const gs_bwd_args* args, hipStream_t stream);
  * args) bytes, 256-byte aligned, zeroed before its first use (like the
  * forward's, it may be shared with forward launches on the same stream), and
  * gs_bwd_scratch_bytes() bytes of scratch. H <= 1024: the reverse recurrence
- * runs on the persistent kernel; 1024 < H <= 8192: on the batch-tiled kernel of
- * gs_dense_bwd_tiled (no workspace; gs_bwd_workspace_bytes() returns 0). */
+ * runs on the persistent kernel, or one launch per step for large batches; 1024 < H <=
+ * 8192: as gs_dense_bwd_tiled's (no workspace; gs_bwd_workspace_bytes() returns 0). */
 int gs_dense_bwd(const gs_bwd_args* args, hipStream_t stream);
 
 /* Barrier-free dense backward (reference gru_scan_backward_triton, scan.py:1355-1447,
  * kernel gru_scan_bwd_kernel, scan.py:916-1352): the passes and products of
- * gs_dense_bwd with the reverse recurrence on a 1-D grid over tiles of batch rows
- * that never wait for each other (Wh transposed once into the scratch, then read
- * from memory every step). No workspace (gs_bwd_workspace_bytes(GS_KIND_DENSE_TILED)
+ * gs_dense_bwd with the reverse recurrence as one launch per step (H >= 129), or on a
+ * 1-D grid over tiles of batch rows that never wait for each other (Wh transposed once
+ * into the scratch, then read from memory every step). No workspace (gs_bwd_workspace_bytes(GS_KIND_DENSE_TILED)
  * is 0), gs_bwd_scratch_bytes(GS_KIND_DENSE_TILED, args) bytes of scratch,
  * 1 <= H <= 8192. Gradients bit-identical to gs_dense_bwd's at H <= 1024. */
 int gs_dense_bwd_tiled(const gs_bwd_args* args, hipStream_t stream);
@@ -565,8 +567,7 @@ int gs_observe_tensor(const gs_observe_tensor_args* args, hipStream_t stream);
 /* The T-step scan with quant_h_in and quant_h_out as observers: at step t,
  * q_in sees h_{t-1} (h0, then out[t-1]; T calls), q_out sees the pre-quant h_t
  * (T calls). Same tensors, strides and hidden-map fields as gs_args; the map
- * is materialized (gs_hidden_map_dense) into the scratch, the steps run as
- * short launches. Forward only. */
+ * is materialized (gs_hidden_map_dense) into the scratch, one launch per step. Forward only. */
 typedef struct gs_observe_args {
   int32_t kind;     /* GS_KIND_*                                                    */
   const float* gi;
