@@ -635,6 +635,49 @@ def _raw_entry(lib: ctypes.CDLL, fn_name: str):
     return fn
 
 
+# The projections' argument structures, packed likewise (layouts of GsProjArgs,
+# GsProjBwdArgs, GsSProjArgs and GsSProjBwdArgs, checked bytewise by the CPU tests).
+PROJ_ARGS = struct.Struct("<7Q5q" "ifii" "ifii" "2Q")
+PROJ_BWD_ARGS = struct.Struct("<8Q7q" "ifii" "2Q" "ifii")
+SPROJ_ARGS = struct.Struct("<i4x8Q9q" "ifii" "ifii" "ifii" "ifii")
+SPROJ_BWD_ARGS = struct.Struct("<i4x10Q10q" "ifii" "ifii" "ifii" "ifii")
+
+
+def raw_size(lib: ctypes.CDLL, fn_name: str, packed: bytes) -> int:
+    """What the size query ``fn_name`` says for packed arguments."""
+    fn = _RAW_FN.get(fn_name)
+    if fn is None:
+        fn = lib[fn_name]
+        fn.argtypes = [ctypes.c_char_p]
+        fn.restype = ctypes.c_int64
+        _RAW_FN[fn_name] = fn
+    n = int(fn(packed))
+    if n < 0:
+        raise_for(n, lib)
+    return n
+
+
+def raw_call(lib: ctypes.CDLL, fn_name: str, packed: bytes, dev: torch.device) -> None:
+    """Calls ``fn_name`` on the current torch stream of ``dev``."""
+    with on_device(dev):
+        rc = _raw_entry(lib, fn_name)(packed, current_stream_handle(dev))
+    raise_for(rc, lib)
+
+
+def quant_fields(mode: int, scale: float, qmin: int, qmax: int) -> tuple:
+    """A gs_quant or gs_oquant as struct fields; bounds past 32 bits wrap, as in a ctypes field."""
+    return (mode, scale, ctypes.c_int32(qmin).value, ctypes.c_int32(qmax).value)
+
+
+def frozen_fields(q: QuantTuple) -> tuple:
+    """A frozen per-tensor (scale, qmin, qmax), or None, as the fields of a gs_quant."""
+    return _QOFF if q is None else quant_fields(1, float(q[0]), int(q[1]), int(q[2]))
+
+
+def ptr(t: Optional[torch.Tensor]) -> int:
+    return t.data_ptr() if t is not None else 0
+
+
 # id(w) -> (weak reference to w, (data_ptr, _version), result); the entry goes
 # when w does. (A WeakKeyDictionary would compare two tensors with ==.)
 _CODES_CACHE: dict = {}

@@ -19,13 +19,12 @@ passing gradient to each row's max and min elements.
 
 from __future__ import annotations
 
-import ctypes
 from typing import Any, Optional, Tuple, cast
 
 import torch
 
 from . import _lib
-from ._common import QuantTuple, check_quant, require_cuda, require_f32
+from ._common import QuantTuple, check_quant, cuda_f32, require_cuda, require_f32
 
 WeightQuant = Optional[Tuple[int, int]]
 
@@ -42,6 +41,10 @@ def _check_wq(w_quant: WeightQuant) -> WeightQuant:
     return (qmin, qmax)
 
 
+def _w_fields(q: WeightQuant) -> tuple:
+    return _lib._QOFF if q is None else _lib.quant_fields(1, 1.0, int(q[0]), int(q[1]))
+
+
 def _project(x2: torch.Tensor, Wi_cat: torch.Tensor, bi_cat: Optional[torch.Tensor], x_quant: QuantTuple,
              w_quant: WeightQuant) -> Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor], Optional[torch.Tensor]]:
     """gi [M, N], the weight used, its per-row scales (or None) and q_x(x) (or None)."""
@@ -49,41 +52,31 @@ def _project(x2: torch.Tensor, Wi_cat: torch.Tensor, bi_cat: Optional[torch.Tens
     M, I = x2.shape
     N = Wi_cat.shape[0]
     gi = torch.empty((M, N), device=x2.device, dtype=x2.dtype)
-    a = _lib.GsProjArgs()
-    a.x, a.w, a.gi = x2.data_ptr(), Wi_cat.data_ptr(), gi.data_ptr()
-    a.bias = bi_cat.data_ptr() if bi_cat is not None else None
-    a.M, a.N, a.I = M, N, I
-    a.sx, a.sgi = x2.stride(0), gi.stride(0)
-    a.q_x = _lib.make_quant(x_quant, "x_quant")
-    xq = None
-    if x_quant is not None:
-        xq = torch.empty((M, I), device=x2.device, dtype=x2.dtype)
-        a.x_q = xq.data_ptr()
+    xq = torch.empty((M, I), device=x2.device, dtype=x2.dtype) if x_quant is not None else None
     w_used, scales = Wi_cat, None
     if w_quant is not None:
         w_used = torch.empty_like(Wi_cat)
         scales = torch.empty((N,), device=x2.device, dtype=x2.dtype)
-        a.w_q, a.w_scale = w_used.data_ptr(), scales.data_ptr()
-        a.q_w = _lib.GsQuant(1, 1.0, int(w_quant[0]), int(w_quant[1]))
-    else:
-        a.q_w = _lib.make_quant(None, "w_quant")
-    codes = None
+    codes, x_codes, w_codes = None, 0, 0
     if (x_quant is not None and w_quant is not None and I % 16 == 0 and int(x_quant[1]) >= -128
             and int(x_quant[2]) <= 127 and w_quant[0] >= -128 and w_quant[1] <= 127):
         # int8 scratch for x's levels and the weight's codes: the product then runs on the int8 MFMA
         codes = torch.empty((M + N) * I, device=x2.device, dtype=torch.int8)
-        a.x_codes, a.w_codes = codes.data_ptr(), codes.data_ptr() + M * I
-    with _lib.on_device(x2.device):
-        rc = lib.gs_input_proj(ctypes.byref(a), ctypes.c_void_p(_lib.current_stream_handle(x2.device)))
-    _lib.raise_for(rc, lib)
+        x_codes = codes.data_ptr()
+        w_codes = x_codes + M * I
+    a = _lib.PROJ_ARGS.pack(x2.data_ptr(), Wi_cat.data_ptr(), _lib.ptr(bi_cat), gi.data_ptr(), _lib.ptr(xq),
+                            w_used.data_ptr() if w_quant is not None else 0, _lib.ptr(scales), M, N, I, x2.stride(0),
+                            gi.stride(0), *_lib.frozen_fields(x_quant), *_w_fields(w_quant), x_codes, w_codes)
+    _lib.raw_call(lib, "gs_input_proj", a, x2.device)
     del codes  # the caching allocator keeps it until the stream's work is done
     return gi, w_used, scales, xq
 
 
 def _validate(who: str, x: torch.Tensor, Wi_cat: torch.Tensor, bi_cat: Optional[torch.Tensor]) -> None:
-    tensors = dict(x=x, Wi_cat=Wi_cat) if bi_cat is None else dict(x=x, Wi_cat=Wi_cat, bi_cat=bi_cat)
-    require_cuda(who, **tensors)
-    require_f32(who, **tensors)
+    if not (cuda_f32(x, Wi_cat) if bi_cat is None else cuda_f32(x, Wi_cat, bi_cat)):
+        tensors = dict(x=x, Wi_cat=Wi_cat) if bi_cat is None else dict(x=x, Wi_cat=Wi_cat, bi_cat=bi_cat)
+        require_cuda(who, **tensors)
+        require_f32(who, **tensors)
     if Wi_cat.dim() != 2 or x.shape[-1] != Wi_cat.shape[1]:
         raise ValueError(f"{who}: Wi_cat must be [N, I] with I = x.shape[-1]={x.shape[-1]}; "
                          f"got {tuple(Wi_cat.shape)}")
@@ -132,25 +125,16 @@ class InputProjectionFunction(torch.autograd.Function):
         dx = torch.empty((M, I), device=x2.device, dtype=x2.dtype)
         dw = torch.empty_like(w_used)
         dbias = torch.empty((N,), device=x2.device, dtype=x2.dtype) if ctx.has_bias else None
-        a = _lib.GsProjBwdArgs()
-        a.x, a.w, a.dgi, a.dx, a.dw = x2.data_ptr(), w_used.data_ptr(), dgi2.data_ptr(), dx.data_ptr(), dw.data_ptr()
-        a.x_q = xq.data_ptr() if xq is not None else None
-        a.dbias = dbias.data_ptr() if dbias is not None else None
-        a.M, a.N, a.I = M, N, I
-        a.sx, a.sdgi, a.sdx = x2.stride(0), dgi2.stride(0), dx.stride(0)
-        a.q_x = _lib.make_quant(ctx.x_quant, "x_quant")
-        if ctx.w_quant is not None:
-            a.w_raw, a.w_scale = w_raw.data_ptr(), scales.data_ptr()
-            a.q_w = _lib.GsQuant(1, 1.0, int(ctx.w_quant[0]), int(ctx.w_quant[1]))
-        need = lib.gs_input_proj_bwd_workspace_bytes(ctypes.byref(a))
-        if need < 0:
-            _lib.raise_for(int(need), lib)
-        ws = torch.empty((max(int(need), 256),), device=x2.device, dtype=torch.uint8)
-        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-        with _lib.on_device(x2.device):
-            rc = lib.gs_input_proj_bwd(ctypes.byref(a),
-                                       ctypes.c_void_p(_lib.current_stream_handle(x2.device)))
-        _lib.raise_for(rc, lib)
+        ptrs = (x2.data_ptr(), w_used.data_ptr(), _lib.ptr(xq), dgi2.data_ptr(), dx.data_ptr(), dw.data_ptr(),
+                _lib.ptr(dbias))
+        w_ptrs = (w_raw.data_ptr(), scales.data_ptr()) if ctx.w_quant is not None else (0, 0)
+        rest = (M, N, I, x2.stride(0), dgi2.stride(0), dx.stride(0), *_lib.frozen_fields(ctx.x_quant), *w_ptrs,
+                *_w_fields(ctx.w_quant))
+        need = _lib.raw_size(lib, "gs_input_proj_bwd_workspace_bytes", _lib.PROJ_BWD_ARGS.pack(*ptrs, 0, 0, *rest))
+        nbytes = max(need, 256)
+        ws = torch.empty((nbytes,), device=x2.device, dtype=torch.uint8)
+        _lib.raw_call(lib, "gs_input_proj_bwd", _lib.PROJ_BWD_ARGS.pack(*ptrs, ws.data_ptr(), nbytes, *rest),
+                      x2.device)
         return dx.view(ctx.x_shape), dw, dbias, None, None
 
 

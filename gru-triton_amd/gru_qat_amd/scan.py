@@ -151,8 +151,9 @@ def _dense_backward(who: str, gi, h0, Wh_cat, bh_cat, out, dout, h_in_quant, h_o
                     gh_saved: Optional[torch.Tensor] = None, tiled: bool = False):
     """Runs gs_dense_bwd (tiled: gs_dense_bwd_tiled); gh_saved is the gh the
     forward stored through gh_save (then the backward skips its recompute GEMM)."""
-    require_cuda(who, gi=gi, h0=h0, Wh_cat=Wh_cat, bh_cat=bh_cat, out=out, dout=dout)
-    require_f32(who, gi=gi, h0=h0, Wh_cat=Wh_cat, bh_cat=bh_cat, out=out, dout=dout)
+    if not cuda_f32(gi, h0, Wh_cat, bh_cat, out, dout):
+        require_cuda(who, gi=gi, h0=h0, Wh_cat=Wh_cat, bh_cat=bh_cat, out=out, dout=dout)
+        require_f32(who, gi=gi, h0=h0, Wh_cat=Wh_cat, bh_cat=bh_cat, out=out, dout=dout)
     T, B, H = check_common(who, gi, h0, bh_cat)
     if tuple(Wh_cat.shape) != (3 * H, H):
         raise ValueError(f"Wh_cat shape must be (3H, H)=({3 * H}, {H}); got {tuple(Wh_cat.shape)}")

@@ -96,8 +96,9 @@ def gru_scan_butterfly_backward(gi, h0, twiddles, bh_cat, out, dout, *, h_in_qua
     comes back as per-row partials summed here.
     """
     who = "gru_scan_butterfly_backward"
-    require_cuda(who, gi=gi, h0=h0, twiddles=twiddles, bh_cat=bh_cat, out=out, dout=dout)
-    require_f32(who, gi=gi, h0=h0, twiddles=twiddles, bh_cat=bh_cat, out=out, dout=dout)
+    if not cuda_f32(gi, h0, twiddles, bh_cat, out, dout):
+        require_cuda(who, gi=gi, h0=h0, twiddles=twiddles, bh_cat=bh_cat, out=out, dout=dout)
+        require_f32(who, gi=gi, h0=h0, twiddles=twiddles, bh_cat=bh_cat, out=out, dout=dout)
     T, B, H = check_common(who, gi, h0, bh_cat)
     nblocks, log_n = check_twiddles(twiddles, H)
     if tuple(out.shape) != (T, B, H) or tuple(dout.shape) != (T, B, H):

@@ -22,7 +22,7 @@ from typing import Any, Tuple, cast
 import torch
 
 from . import _lib
-from ._common import QuantTuple, check_common, check_quant, require_cuda, require_f32
+from ._common import QuantTuple, check_common, check_quant, cuda_f32, require_cuda, require_f32
 from .observe import hidden_map_dense, hidden_map_grad
 from .scan import gru_scan_backward_persistent, gru_scan_forward_persistent
 
@@ -42,8 +42,9 @@ def extract_circulant_factors(cell: Any) -> Tuple[torch.Tensor, torch.Tensor]:
 
 
 def _check(who: str, gi, h0, Wh_circ, bh_cat) -> int:
-    require_cuda(who, gi=gi, h0=h0, Wh_circ=Wh_circ, bh_cat=bh_cat)
-    require_f32(who, gi=gi, h0=h0, Wh_circ=Wh_circ, bh_cat=bh_cat)
+    if not cuda_f32(gi, h0, Wh_circ, bh_cat):
+        require_cuda(who, gi=gi, h0=h0, Wh_circ=Wh_circ, bh_cat=bh_cat)
+        require_f32(who, gi=gi, h0=h0, Wh_circ=Wh_circ, bh_cat=bh_cat)
     _, _, H = check_common(who, gi, h0, bh_cat)
     if tuple(Wh_circ.shape) != (3, H):
         raise ValueError(f"Wh_circ shape must be (3, H)=(3, {H}); got {tuple(Wh_circ.shape)}")

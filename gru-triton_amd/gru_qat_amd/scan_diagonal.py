@@ -70,8 +70,9 @@ def gru_scan_diagonal_backward(gi, h0, Wh_diag, bh_cat, out, dout, *, h_in_quant
     summed over B here.
     """
     who = "gru_scan_diagonal_backward"
-    require_cuda(who, gi=gi, h0=h0, Wh_diag=Wh_diag, bh_cat=bh_cat, out=out, dout=dout)
-    require_f32(who, gi=gi, h0=h0, Wh_diag=Wh_diag, bh_cat=bh_cat, out=out, dout=dout)
+    if not cuda_f32(gi, h0, Wh_diag, bh_cat, out, dout):
+        require_cuda(who, gi=gi, h0=h0, Wh_diag=Wh_diag, bh_cat=bh_cat, out=out, dout=dout)
+        require_f32(who, gi=gi, h0=h0, Wh_diag=Wh_diag, bh_cat=bh_cat, out=out, dout=dout)
     T, B, H = check_common(who, gi, h0, bh_cat)
     if tuple(out.shape) != (T, B, H) or tuple(dout.shape) != (T, B, H):
         raise ValueError(f"out and dout must be (T, B, H)=({T}, {B}, {H})")

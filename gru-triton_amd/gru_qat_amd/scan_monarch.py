@@ -124,8 +124,9 @@ def gru_scan_monarch_backward(gi, h0, Wh_struct, bh_cat, out, dout, *, h_in_quan
     gh_saved (what the forward stored through gh_save), skips its gh product.
     """
     who = "gru_scan_monarch_backward"
-    require_cuda(who, gi=gi, h0=h0, Wh_struct=Wh_struct, bh_cat=bh_cat, out=out, dout=dout)
-    require_f32(who, gi=gi, h0=h0, Wh_struct=Wh_struct, bh_cat=bh_cat, out=out, dout=dout)
+    if not cuda_f32(gi, h0, Wh_struct, bh_cat, out, dout):
+        require_cuda(who, gi=gi, h0=h0, Wh_struct=Wh_struct, bh_cat=bh_cat, out=out, dout=dout)
+        require_f32(who, gi=gi, h0=h0, Wh_struct=Wh_struct, bh_cat=bh_cat, out=out, dout=dout)
     T, B, H = check_common(who, gi, h0, bh_cat)
     nblocks, blksz = _check_struct("Wh_struct", Wh_struct, H)
     if Wh_struct2 is not None:

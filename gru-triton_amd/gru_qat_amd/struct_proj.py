@@ -26,32 +26,32 @@ path included.
 
 from __future__ import annotations
 
-import ctypes
 from typing import Any, Optional, Sequence, Tuple, cast
 
 import torch
 
 from . import _lib
-from ._common import QuantTuple, check_quant, require_cuda, require_f32
+from ._common import QuantTuple, check_quant, cuda_f32, require_cuda, require_f32
 
 INPUT_KINDS = {"diagonal": _lib.KIND_DIAGONAL, "monarch": _lib.KIND_MONARCH, "butterfly": _lib.KIND_BUTTERFLY}
 OQ_OFF, OQ_FROZEN, OQ_ROWS = 0, 1, 2
 
 
-def _oquant(spec: Any, gate: str) -> _lib.GsOQuant:
+def _oquant(spec: Any, gate: str) -> tuple:
+    """One gate's output quantizer as the fields (mode, scale, qmin, qmax) of a gs_oquant."""
     if spec is None:
-        return _lib.GsOQuant(OQ_OFF, 1.0, 0, 0)
+        return (OQ_OFF, 1.0, 0, 0)
     if isinstance(spec, (tuple, list)) and len(spec) == 3 and spec[0] == "rows":
         qmin, qmax = int(spec[1]), int(spec[2])
         if not (qmax > 0 and qmin <= qmax):
             raise ValueError(f"out_quant[{gate}] ('rows', qmin, qmax) needs qmax > 0 and qmin <= qmax; got {spec!r}")
-        return _lib.GsOQuant(OQ_ROWS, 1.0, qmin, qmax)
+        return _lib.quant_fields(OQ_ROWS, 1.0, qmin, qmax)
     q = check_quant(spec, f"out_quant[{gate}]")
     assert q is not None
-    return _lib.GsOQuant(OQ_FROZEN, float(q[0]), int(q[1]), int(q[2]))
+    return _lib.quant_fields(OQ_FROZEN, float(q[0]), int(q[1]), int(q[2]))
 
 
-def _oquants(out_quant: Any) -> Tuple[_lib.GsOQuant, _lib.GsOQuant, _lib.GsOQuant]:
+def _oquants(out_quant: Any) -> Tuple[tuple, tuple, tuple]:
     if out_quant is None:
         specs: Sequence[Any] = (None, None, None)
     elif isinstance(out_quant, (tuple, list)) and len(out_quant) == 3 and not isinstance(out_quant[0], (int, float, str)):
@@ -83,10 +83,6 @@ def struct_dims(kind: str, W: torch.Tensor, H: int) -> Tuple[int, int, int, int]
     raise ValueError(f"structured input kind must be one of {sorted(INPUT_KINDS)}; got {kind!r}")
 
 
-def _stream(dev: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(_lib.current_stream_handle(dev))
-
-
 class StructInputProjFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx: Any, x, W, bias, kind, x_quant, out_quant):  # type: ignore[override]
@@ -98,33 +94,20 @@ class StructInputProjFunction(torch.autograd.Function):
         M = x2.shape[0]
         nb, bs, L, nch = struct_dims(kind, W, H)
         oq = _oquants(out_quant)
-        any_oq = any(o.mode != OQ_OFF for o in oq)
-        any_rows = any(o.mode == OQ_ROWS for o in oq)
+        any_oq = any(o[0] != OQ_OFF for o in oq)
+        any_rows = any(o[0] == OQ_ROWS for o in oq)
         dev = x2.device
         gi = torch.empty((M, 3 * H), device=dev, dtype=x2.dtype)
         y = torch.empty((M, 3 * H), device=dev, dtype=x2.dtype) if any_oq else None
         y_scale = torch.empty((3, M), device=dev, dtype=x2.dtype) if any_rows else None
         xq = torch.empty((M, H), device=dev, dtype=x2.dtype) if x_quant is not None else None
-        a = _lib.GsSProjArgs()
-        a.kind = INPUT_KINDS[kind]
-        a.x, a.w, a.gi = x2.data_ptr(), W.data_ptr(), gi.data_ptr()
-        a.bias = bias.data_ptr() if bias is not None else None
-        a.y = y.data_ptr() if y is not None else None
-        a.y_scale = y_scale.data_ptr() if y_scale is not None else None
-        a.x_q = xq.data_ptr() if xq is not None else None
-        a.M, a.H, a.sx, a.sgi = M, H, x2.stride(0), gi.stride(0)
-        a.nblocks, a.blksz, a.log_n, a.bfly_nblocks = nb, bs, L, nch
-        a.q_x = _lib.make_quant(x_quant, "x_quant")
-        for g in range(3):
-            a.q_out[g] = oq[g]
-        need = lib.gs_struct_input_proj_scratch_bytes(ctypes.byref(a))
-        if need < 0:
-            _lib.raise_for(int(need), lib)
-        scratch = torch.empty((max(int(need), 256),), device=dev, dtype=torch.uint8)
-        a.scratch, a.scratch_bytes = scratch.data_ptr(), scratch.numel()
-        with _lib.on_device(dev):
-            rc = lib.gs_struct_input_proj(ctypes.byref(a), _stream(dev))
-        _lib.raise_for(rc, lib)
+        ptrs = (INPUT_KINDS[kind], x2.data_ptr(), W.data_ptr(), _lib.ptr(bias), gi.data_ptr(), _lib.ptr(y),
+                _lib.ptr(y_scale), _lib.ptr(xq))
+        rest = (M, H, x2.stride(0), gi.stride(0), nb, bs, L, nch, *_lib.frozen_fields(x_quant), *oq[0], *oq[1], *oq[2])
+        need = _lib.raw_size(lib, "gs_struct_input_proj_scratch_bytes", _lib.SPROJ_ARGS.pack(*ptrs, 0, 0, *rest))
+        nbytes = max(need, 256)
+        scratch = torch.empty((nbytes,), device=dev, dtype=torch.uint8)
+        _lib.raw_call(lib, "gs_struct_input_proj", _lib.SPROJ_ARGS.pack(*ptrs, scratch.data_ptr(), nbytes, *rest), dev)
         ctx.save_for_backward(x2, W, xq, y, y_scale)
         ctx.kind, ctx.x_quant, ctx.oq = kind, x_quant, oq
         ctx.dims = (nb, bs, L, nch)
@@ -144,26 +127,17 @@ class StructInputProjFunction(torch.autograd.Function):
         dx = torch.empty((M, H), device=dev, dtype=x2.dtype)
         dW = torch.empty_like(W)
         dbias = torch.empty((3 * H,), device=dev, dtype=x2.dtype) if ctx.has_bias else None
-        a = _lib.GsSProjBwdArgs()
-        a.kind = INPUT_KINDS[ctx.kind]
-        a.x, a.w, a.dgi, a.dx, a.dw = x2.data_ptr(), W.data_ptr(), dgi2.data_ptr(), dx.data_ptr(), dW.data_ptr()
-        a.x_q = xq.data_ptr() if xq is not None else None
-        a.y = y.data_ptr() if y is not None else None
-        a.y_scale = y_scale.data_ptr() if y_scale is not None else None
-        a.dbias = dbias.data_ptr() if dbias is not None else None
-        a.M, a.H, a.sx, a.sdgi, a.sdx = M, H, x2.stride(0), dgi2.stride(0), dx.stride(0)
-        a.nblocks, a.blksz, a.log_n, a.bfly_nblocks = ctx.dims
-        a.q_x = _lib.make_quant(ctx.x_quant, "x_quant")
-        for g in range(3):
-            a.q_out[g] = ctx.oq[g]
-        need = lib.gs_struct_input_proj_bwd_scratch_bytes(ctypes.byref(a))
-        if need < 0:
-            _lib.raise_for(int(need), lib)
-        scratch = torch.empty((max(int(need), 256),), device=dev, dtype=torch.uint8)
-        a.scratch, a.scratch_bytes = scratch.data_ptr(), scratch.numel()
-        with _lib.on_device(dev):
-            rc = lib.gs_struct_input_proj_bwd(ctypes.byref(a), _stream(dev))
-        _lib.raise_for(rc, lib)
+        ptrs = (INPUT_KINDS[ctx.kind], x2.data_ptr(), _lib.ptr(xq), W.data_ptr(), _lib.ptr(y), _lib.ptr(y_scale),
+                dgi2.data_ptr(), dx.data_ptr(), dW.data_ptr(), _lib.ptr(dbias))
+        oq = ctx.oq
+        rest = (M, H, x2.stride(0), dgi2.stride(0), dx.stride(0), *ctx.dims, *_lib.frozen_fields(ctx.x_quant), *oq[0], *oq[1],
+                *oq[2])
+        need = _lib.raw_size(lib, "gs_struct_input_proj_bwd_scratch_bytes",
+                             _lib.SPROJ_BWD_ARGS.pack(*ptrs, 0, 0, *rest))
+        nbytes = max(need, 256)
+        scratch = torch.empty((nbytes,), device=dev, dtype=torch.uint8)
+        _lib.raw_call(lib, "gs_struct_input_proj_bwd",
+                      _lib.SPROJ_BWD_ARGS.pack(*ptrs, scratch.data_ptr(), nbytes, *rest), dev)
         return dx.view(ctx.x_shape), dW, dbias, None, None, None
 
 
@@ -174,9 +148,10 @@ def structured_input_projection(x: torch.Tensor, kind: str, Wi_struct: torch.Ten
     input side ``kind`` with stacked weights ``Wi_struct``; differentiable in
     x, Wi_struct and bi_cat."""
     who = "structured_input_projection"
-    tensors = dict(x=x, Wi_struct=Wi_struct) if bi_cat is None else dict(x=x, Wi_struct=Wi_struct, bi_cat=bi_cat)
-    require_cuda(who, **tensors)
-    require_f32(who, **tensors)
+    if not (cuda_f32(x, Wi_struct) if bi_cat is None else cuda_f32(x, Wi_struct, bi_cat)):
+        tensors = dict(x=x, Wi_struct=Wi_struct) if bi_cat is None else dict(x=x, Wi_struct=Wi_struct, bi_cat=bi_cat)
+        require_cuda(who, **tensors)
+        require_f32(who, **tensors)
     if kind not in INPUT_KINDS:
         raise ValueError(f"{who}: kind must be one of {sorted(INPUT_KINDS)}; got {kind!r}")
     if x.dim() < 1 or x.numel() == 0:
