@@ -674,6 +674,14 @@ bool overlap(const float* a, int64_t an, const float* b, int64_t bn) { return a 
 constexpr int64_t kStepMinH = 129;
 constexpr int64_t kStepMaxB = 16 * 65535;  // 16-row tiles in the grid's second dimension
 
+// A training step is some 120 to 160 us of host time, behind which a few steps
+// of few units run on one CU for nothing, while a launch each adds 2.5 us to it.
+// Forward and backward, us, one-CU kernels / launches: T = 8, B = 4, H = 140
+// 152 / 173; T = 6, B = 32, H = 200 176 / 189; T = 10, B = 16, H = 160 208 / 212;
+// T = 3, B = 16, H = 320 164 / 171 (T H^2 = 157000 to 307000); T = 10, B = 2, H = 361
+// 1120 / 204. So training scans take launches from T H^2 = 400000 on, or for one step.
+bool enough_steps(int64_t T, int64_t H) { return T == 1 || T * H * H >= 400000; }
+
 }  // namespace
 
 // The step kernels address a workgroup's state rows (at most 64) with 32-bit
@@ -682,6 +690,7 @@ constexpr int64_t kStepMaxB = 16 * 65535;  // 16-row tiles in the grid's second 
 // batch tile's steps by itself allows (scan_tiled.hip).
 bool step_fwd_applies(const gs_args* a) {
   if (a->H < kStepMinH || a->B > kStepMaxB) return false;
+  if (a->gh_save != nullptr && !enough_steps(a->T, a->H)) return false;
   if (a->B > 1 && std::max(a->sh0_b, a->so_b) > int64_t(1) << 22) return false;
   const int64_t n_out = (a->T - 1) * a->so_t + (a->B - 1) * a->so_b + a->H;
   const int64_t n_gi = (a->T - 1) * a->sg_t + (a->B - 1) * a->sg_b + 3 * a->H;
@@ -727,13 +736,9 @@ bool step_bwd_beats_persistent(int64_t T, int64_t B, int64_t H) {
   return kc >= 16 && B <= kStepMaxB && rounds >= least && pays_launches(T, rounds);
 }
 
-// dh0 is written by the launch that reads D_0, and dout is D_{T-1}. A few steps
-// of few units are over before the host has queued a launch each (T = 3, B = 5,
-// H = 66, a training step that the host bounds: 152 us with the one-CU kernel,
-// 162 with launches), so two steps or more take launches from T H^2 = 200000
-// on (about 30 us of the one-CU kernel).
+// dh0 is written by the launch that reads D_0, and dout is D_{T-1}.
 bool step_bwd_applies(const float* dout, const float* dh0, int64_t T, int64_t B, int64_t H) {
-  return H >= kStepMinH && B <= kStepMaxB && (T == 1 || T * H * H >= 200000) && !overlap(dh0, B * H, dout, T * B * H);
+  return H >= kStepMinH && B <= kStepMaxB && enough_steps(T, H) && !overlap(dh0, B * H, dout, T * B * H);
 }
 
 // The forward, one launch per step (see the header comment).

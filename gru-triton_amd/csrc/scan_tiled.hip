@@ -13,8 +13,8 @@
 // is served by one launch per step over all CUs (scan_step.hip): a step here
 // streams all of Wh through each tile's one CU, 2.9 us at H = 64 against 3.6 us
 // for a launch, but 12 against 4 at H = 192, 60 against 6 at H = 512 and 990
-// against 14.6 at H = 2048 (B = 32). These kernels run up to 128 units, in the
-// backward also a few steps of a few hundred, and at any H where a launch per
+// against 14.6 at H = 2048 (B = 32). These kernels run up to 128 units, in
+// training also a few steps of a few hundred, and at any H where a launch per
 // step cannot: tensors that overlap (step_fwd_applies, step_bwd_applies).
 //
 // Work split. A workgroup of 8 waves owns BT <= 4 batch rows. Per step each

@@ -19,9 +19,9 @@ pytestmark = pytest.mark.gpu
 
 OTHER = (0.05, -10, 10)
 # (T, B, H): 129 the smallest H; 16 / 17 and 64 / 65 rows; K one past and one short of a chunk; rows of every
-# length modulo 4; T H^2 on both sides of the backward's bound; 32 and 64 rows a workgroup (B = 90 x 1000,
+# length modulo 4; T H^2 on both sides of the training scans' bound; 32 and 64 rows a workgroup (B = 90 x 1000,
 # B = 250 x 1024)
-SHAPES = [(13, 1, 129), (11, 16, 130), (3, 17, 191), (4, 65, 257), (1, 33, 192), (3, 90, 1000), (2, 250, 1024)]
+SHAPES = [(13, 1, 129), (25, 1, 129), (11, 16, 130), (24, 17, 131), (7, 65, 257), (3, 17, 191), (4, 65, 257), (1, 33, 192), (3, 90, 1000), (2, 250, 1024)]
 
 
 def _cfg(shape, q_in=None, q_out=None, int8=False):
