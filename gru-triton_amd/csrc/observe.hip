@@ -337,7 +337,7 @@ __device__ __forceinline__ void step_scales(const OStep& p, StepIn& v, DynQuant*
       scale_zp(p.c.out, mn, mx, &s_out, &zp_out);
       if (writer) {
         observe_in(p.c.out, v.out, mn, mx);
-        if (p.c.in.stats == p.c.out.stats) {  // one quantizer in both places
+        if (p.c.out.mode == GS_OBS_MIN_MAX && p.c.in.stats == p.c.out.stats) {  // one quantizer in both places
 #pragma unroll
           for (int j = 0; j < 3; ++j) v.in[j] = v.out[j];
         }

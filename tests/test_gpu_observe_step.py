@@ -6,11 +6,14 @@ test_gpu_observe.py."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
 import gru_qat_amd as G
 from oracle import gru_oracle as O
+from parity_util import to_dev
 from test_gpu_observe import _cfg, _codes_match, _quant, _run, _teacher_forced
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +68,40 @@ def test_observe_one_side_off(dev, idx, which):
             assert abs(float(trace[t, 2]) - s) <= 1e-5 * s
             _codes_match(out[t], pre, float(trace[t, 2]), 0.0, -127, 127)
     assert torch.allclose(q.observer_stats.cpu()[:2], torch.stack([st.running_min, st.running_max]), rtol=1e-5)
+
+
+def _observe_raw(dev, kind, gi, h0, w, bh, q_in, q_out):
+    """gs_observe_scan on device tensors with the C ABI's own observers."""
+    from gru_qat_amd import _lib
+
+    lib = _lib.load()
+    T, B, H3 = gi.shape
+    out = torch.empty((T, B, H3 // 3), device=dev)
+    a = _lib.GsObserveArgs(kind=kind, gi=gi.data_ptr(), h0=h0.data_ptr(), w=w.data_ptr(), bh=bh.data_ptr(),
+                           out=out.data_ptr(), T=T, B=B, H=H3 // 3, sg_t=gi.stride(0), sg_b=gi.stride(1),
+                           sh0_b=h0.stride(0), so_t=out.stride(0), so_b=out.stride(1), q_in=q_in, q_out=q_out)
+    need = lib.gs_observe_scan_scratch_bytes(ctypes.byref(a))
+    _lib.raise_for(min(need, 0), lib)
+    scratch = torch.empty(int(need), dtype=torch.uint8, device=dev)
+    a.scratch, a.scratch_bytes = scratch.data_ptr(), scratch.numel()
+    _lib.raise_for(lib.gs_observe_scan(ctypes.byref(a), ctypes.c_void_p(_lib.current_stream_handle(dev))), lib)
+    torch.cuda.synchronize(dev)
+    return out
+
+
+@pytest.mark.parametrize("idx", [0, 1])
+def test_observe_shared_stats_pointer_with_other_modes(dev, idx):
+    """A dynamic q_out keeps no statistics, so a stats pointer that it shares with a min_max q_in is q_in's alone."""
+    from gru_qat_amd import _lib
+
+    cfg = _cfg(idx, (4, 5, 96))
+    d = to_dev(cfg, dev)
+    got = []
+    for shared in (False, True):
+        stats = torch.tensor([float("inf"), float("-inf"), 0.0], device=dev)
+        q_in = _lib.GsObserver(_lib.OBS_MIN_MAX, 1, -127, 127, 1.0, 0.0, stats.data_ptr())
+        q_out = _lib.GsObserver(_lib.OBS_DYNAMIC, 1, -127, 127, 1.0, 0.0, stats.data_ptr() if shared else None)
+        kind = _lib.KIND_DIAGONAL if idx == 0 else _lib.KIND_DENSE
+        got.append((_observe_raw(dev, kind, d["gi"], d["h0"], d["w"], d["bh"], q_in, q_out), stats))
+    assert torch.equal(got[0][0], got[1][0])
+    assert torch.equal(got[0][1], got[1][1]), (got[0][1].tolist(), got[1][1].tolist())
