@@ -228,7 +228,9 @@ __global__ __launch_bounds__(kRedThreads) void quant_step(const float2* part, in
 // ---- one step ------------------------------------------------------------------------
 
 // fq at a scale found at run time. A symmetric one in quant_code's range takes
-// its division-free quotient, which equals the IEEE one (gs_device.h).
+// its division-free quotient, which equals the IEEE one (gs_device.h). Codes stay
+// below 2^22 there: the bound under which q_in repeats q_out (same_quant,
+// gs_host.h), inside the 2^24 up to which the quotient holds.
 struct DynQuant {
   Quant q;
   float zp;
@@ -246,7 +248,8 @@ struct DynQuant {
 
 __device__ __forceinline__ DynQuant dyn_quant(const Obs& o, float s, float zp) {
   DynQuant d{{s, o.qmin, o.qmax, 1, 1.0f / s}, zp, o.mode != GS_OBS_OFF, 0};
-  d.fast = d.on && zp == 0.0f && s >= 0x1p-126f && s <= 0x1p64f;
+  d.fast = d.on && zp == 0.0f && s >= 0x1p-126f && s <= 0x1p64f && o.qmin >= -0x1p22f &&
+           o.qmax <= 0x1p22f;
   return d;
 }
 

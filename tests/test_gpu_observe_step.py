@@ -105,3 +105,24 @@ def test_observe_shared_stats_pointer_with_other_modes(dev, idx):
         got.append((_observe_raw(dev, kind, d["gi"], d["h0"], d["w"], d["bh"], q_in, q_out), stats))
     assert torch.equal(got[0][0], got[1][0])
     assert torch.equal(got[0][1], got[1][1]), (got[0][1].tolist(), got[1][1].tolist())
+
+
+@pytest.mark.parametrize("idx", [0, 1])
+@pytest.mark.parametrize("mode", ["frozen", "dynamic"])
+def test_observe_codes_past_24_bits(dev, idx, mode):
+    """Ranges past the bound of the division-free quotient take the IEEE one: out[0], which the launch of step 1
+    quantizes, is fake_quant_ste's of the pre-quant state bit for bit."""
+    from gru_qat_amd import _lib
+
+    T, B, H = 2, 37, 64
+    cfg = _cfg(idx, (T, B, H))
+    d = to_dev(cfg, dev)
+    args = (_lib.KIND_DIAGONAL if idx == 0 else _lib.KIND_DENSE, d["gi"], d["h0"], d["w"], d["bh"])
+    off = _lib.GsObserver(_lib.OBS_OFF, 1, 0, 1, 1.0, 0.0, None)
+    pre = _observe_raw(dev, *args, off, off)[0].cpu()
+    lim = 2 ** 30
+    s = torch.tensor(1e-9) if mode == "frozen" else pre.abs().max().clamp(min=1e-8) / torch.tensor(float(lim))
+    q_out = _lib.GsObserver(_lib.OBS_FROZEN if mode == "frozen" else _lib.OBS_DYNAMIC, 1, -lim, lim, 1e-9, 0.0, None)
+    out = _observe_raw(dev, *args, off, q_out)[0].cpu()
+    ref = torch.round(pre / s).clamp(-lim, lim) * s
+    assert torch.equal(out, ref), f"{int((out != ref).sum())} of {ref.numel()} differ"
