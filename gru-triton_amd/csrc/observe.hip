@@ -24,6 +24,9 @@
 //              partial of its part of the pre-quant h_t. out[t-1] = q_out(h_{t-1})
 //              is written on the way by the workgroup that owns the element.
 //   at last:   out[T-1] = q_out(h_{T-1}).
+// Batches whose step would be several rounds of workgroups take three launches a
+// step instead (one_launch): the product by gemm.hip with K split, the gates, and a
+// quantizer pass, which fill the CUs better there. Same bits either way.
 // fq is monotone, so the min and max of q_out(h_{t-1}), which q_in sees at step
 // t, are q_out of the pre-quant min and max: one reduction per step covers
 // both quantizers.
@@ -40,7 +43,7 @@ namespace {
 
 constexpr int kRedThreads = 256;
 constexpr int kMaxParts = 512;  // (min, max) partials of one reduction
-constexpr int kMaxSplit = 8;    // K splits of a step's product, one wave each
+constexpr int kMaxSplit = 8;    // K splits of a step's product (one wave each in observe_step_kernel)
 // _update_observer's mixing weights as the fp32 values torch multiplies by.
 constexpr float kKeep = (float)0.99;
 constexpr float kMix = (float)(1.0 - 0.99);
@@ -223,6 +226,39 @@ __global__ __launch_bounds__(kRedThreads) void quant_step(const float2* part, in
     if (dst != nullptr) dst[r * ldd + k] = v;
     if (hq != nullptr) hq[e] = fq(v, s_in, zp_in, c.in.qmin, c.in.qmax);
   }
+}
+
+// The gates of one step of the three-launch form; writes the pre-quant h_t to
+// out_t and a (min, max) partial per workgroup. gh comes from `nsplit` GEMM
+// partials [B, 3H] (split 0 holds the bias).
+__global__ __launch_bounds__(kRedThreads) void gates_step(const float* gi_t, int64_t sg_b, const float* gh, int nsplit,
+                                                          int64_t split_stride, const float* hprev, int64_t shp_b,
+                                                          float* out_t, int64_t so_b, int B, int H, float2* part) {
+  float mn = __builtin_inff(), mx = -__builtin_inff();
+  const int64_t n = (int64_t)B * H;
+  for (int64_t e = blockIdx.x * (int64_t)kRedThreads + threadIdx.x; e < n; e += (int64_t)gridDim.x * kRedThreads) {
+    const int b = (int)(e / H), k = (int)(e - (int64_t)b * H);
+    const float* p = gh + (int64_t)b * 3 * H + k;
+    float v[kMaxSplit][3], g3[3];
+#pragma unroll
+    for (int q = 0; q < kMaxSplit; ++q)
+#pragma unroll
+      for (int g = 0; g < 3; ++g) v[q][g] = q < nsplit ? p[q * split_stride + g * H] : 0.0f;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      float sum = v[0][g];
+#pragma unroll
+      for (int q = 1; q < kMaxSplit; ++q)
+        if (q < nsplit) sum += v[q][g];
+      g3[g] = sum;
+    }
+    const float* gr = gi_t + (int64_t)b * sg_b + k;
+    const float h = gru_update(gr[0], gr[H], gr[2 * H], g3[0], g3[1], g3[2], hprev[(int64_t)b * shp_b + k]);
+    out_t[(int64_t)b * so_b + k] = h;
+    mn = __builtin_fminf(mn, h);
+    mx = __builtin_fmaxf(mx, h);
+  }
+  block_minmax(mn, mx, part + blockIdx.x);
 }
 
 // ---- one step ------------------------------------------------------------------------
@@ -587,18 +623,6 @@ __global__ __launch_bounds__(kRedThreads) void observe_diag_kernel(OStep p) {
   wg_minmax<kRedThreads / 64>(mn, mx, red2, p.part_out + blockIdx.x);
 }
 
-// One (min, max) from n: a step of very many workgroups, whose partials every
-// workgroup of the next would read.
-__global__ __launch_bounds__(1024) void reduce_partials_kernel(const float2* part, int n, float2* dst) {
-  __shared__ float2 red2[16];
-  float mn = __builtin_inff(), mx = -__builtin_inff();
-  for (int i = threadIdx.x; i < n; i += 1024) {
-    mn = __builtin_fminf(mn, part[i].x);
-    mx = __builtin_fmaxf(mx, part[i].y);
-  }
-  wg_minmax<16>(mn, mx, red2, dst);
-}
-
 int validate_observer(const gs_observer& o, const char* name, const char* who) {
   if (o.mode < GS_OBS_OFF || o.mode > GS_OBS_MIN_MAX)
     return set_error(GS_ERR_INVALID, "%s: %s mode %d is not a GS_OBS_* value", who, name, o.mode);
@@ -632,16 +656,32 @@ dim3 grid1d(int64_t n) { return dim3((unsigned)std::min<int64_t>((n + 255) / 256
 
 // Scratch of gs_observe_scan, each region 256-byte aligned:
 // scales [4] | partials of two steps | pre-quant h of two steps [2][B, H] (not
-// the diagonal kind) | map [3H, H] (Monarch, butterfly, circulant) | map
-// construction scratch.
+// the diagonal kind), or with three launches a step hq [B, H] and gh [split][B, 3H] |
+// map [3H, H] (Monarch, butterfly, circulant) | map construction scratch.
 struct OPlan {
   bool gemm, own_map;
+  bool three;   // three launches a step
   int split;
   int rt;       // 16-row tiles a workgroup (1 or 2)
   int64_t nwg;  // workgroups, and partials, of a step
-  int64_t st, part, hpre, map, map_tmp;
-  int64_t total() const { return st + 2 * part + 2 * hpre + map + map_tmp; }
+  int64_t st, part, hpre, gh, map, map_tmp;
+  int64_t total() const { return st + 2 * part + (three ? 1 : 2) * hpre + gh + map + map_tmp; }
 };
+
+// Whether a step of the kinds with a product is one launch. Up to a workgroup per
+// CU always; a further round costs as much again (an 8-wave workgroup holds a CU's
+// LDS), which pays while the eight waves share K without a rest and the product is
+// short. us a step, three launches / one: one round 13 to 83 / 6 to 48; two rounds
+// H = 64, B = 4096 18.6 / 16.5, H = 512, B = 512 31.9 / 22.9, H = 2048, B = 128 57 / 52, but
+// H = 100, B = 2048 18.1 / 22.3, H = 640, B = 256 27.0 / 29.8, H = 3072, B = 64 50 / 70; three
+// H = 192, B = 2048 28.6 / 26.7, H = 1024, B = 384 53.5 / 47.4, but H = 16, B = 20000 19.1 / 22.9;
+// four and more H = 64, B = 20000 38 / 62, H = 127, B = 8192 37 / 83, H = 512, B = 1024 46.9 / 46.1.
+bool one_launch(int64_t H, int split, int64_t nwg) {
+  const int64_t rounds = (nwg + 255) / 256;
+  if (rounds <= 1) return true;
+  if (H % (64 * split) != 0) return false;
+  return rounds == 2 ? H <= 2048 : rounds == 3 && H >= 192 && H <= 1024;
+}
 
 gs_map_args map_view(const gs_observe_args* a) {
   gs_map_args m{};
@@ -686,17 +726,67 @@ int plan_observe(const gs_observe_args* a, OPlan* p, const char* who) {
     return set_error(GS_ERR_INVALID, "%s: B * 3H = %lld is too large", who, (long long)(B * 3 * H));
   p->gemm = a->kind != GS_KIND_DIAGONAL;
   p->own_map = a->kind == GS_KIND_MONARCH || a->kind == GS_KIND_BUTTERFLY || a->kind == GS_KIND_CIRCULANT;
-  // gh has only B rows: split K in up to 8 parts of >= 64 terms, one wave each
+  // gh has only B rows: split K in up to 8 parts of >= 64 terms
   p->split = p->gemm ? (int)std::max<int64_t>(1, std::min<int64_t>(kMaxSplit, H / 64)) : 1;
   // 32 rows a workgroup (Wh read half as often) once 16 give every CU one
   const int64_t nut = (H + 15) / 16;
   p->rt = ((B + 15) / 16) * nut > 256 ? 2 : 1;
   p->nwg = p->gemm ? ((B + 16 * p->rt - 1) / (16 * p->rt)) * nut : parts_for(B * H);
+  p->three = p->gemm && !one_launch(H, p->split, p->nwg);
+  if (p->three) p->nwg = parts_for(B * H);
   p->st = 256;
   p->part = align256(std::max<int64_t>(p->nwg, kMaxParts) * 8);
   p->hpre = p->gemm ? align256(B * H * 4) : 0;
+  p->gh = p->three ? align256((int64_t)p->split * B * 3 * H * 4) : 0;
   p->map = p->own_map ? align256(3 * H * H * 4) : 0;
   p->map_tmp = p->own_map ? hidden_map_scratch(&m) : 0;
+  return GS_OK;
+}
+
+// The steps as three launches each: gh by the K-split GEMM from hq = q_in(h_{t-1}),
+// the gates (pre-quant h_t into out[t]), and a quantizer pass that finishes out[t]
+// and writes the next step's hq. part: kMaxParts partials; those of h0 are in it.
+int three_launches(const gs_observe_args* a, const OPlan& p, const ObsPair& c, const float* W, float* st, float2* part,
+                   float* hq, float* gh, hipStream_t stream, const char* who) {
+  const int T = (int)a->T, B = (int)a->B, H = (int)a->H;
+  const int64_t BH = (int64_t)B * H;
+  const bool in_on = c.in.mode != GS_OBS_OFF, out_on = c.out.mode != GS_OBS_OFF;
+  const int np = is_dynamic(c.in) || is_dynamic(c.out) ? (int)p.nwg : 0;
+  if (in_on) {
+    hipLaunchKernelGGL(quant_step, grid1d(BH), dim3(kRedThreads), 0, stream, part, is_dynamic(c.in) ? (int)p.nwg : 0,
+                       c, st, a->trace, 0, T, 0, a->h0, a->sh0_b, nullptr, (int64_t)0, hq, (int64_t)B, H, 0);
+    GS_CHECK_HIP(hipGetLastError());
+  }
+  for (int t = 0; t < T; ++t) {
+    const float* hprev = t == 0 ? a->h0 : a->out + (int64_t)(t - 1) * a->so_t;
+    const int64_t shp = t == 0 ? a->sh0_b : a->so_b;
+    float* out_t = a->out + (int64_t)t * a->so_t;
+    GemmArgs g;
+    g.a = in_on ? hq : hprev;  // the matmul-side h
+    g.lda = in_on ? H : shp;
+    g.b = W;  // B(k, n) = W[n][k]
+    g.ldb = H;
+    g.c = gh;
+    g.ldc = 3 * H;
+    g.split_stride = 3 * BH;
+    g.bias = a->bh;
+    g.M = B;
+    g.N = 3 * H;
+    g.K = H;
+    g.ksplit = p.split;
+    g.layout = kGemmNT;
+    const int rc = gemm_f32(g, stream, who);
+    if (rc) return rc;
+    hipLaunchKernelGGL(gates_step, dim3((unsigned)p.nwg), dim3(kRedThreads), 0, stream,
+                       a->gi + (int64_t)t * a->sg_t, a->sg_b, gh, p.split, 3 * BH, hprev, shp, out_t, a->so_b, B, H,
+                       part);
+    GS_CHECK_HIP(hipGetLastError());
+    // every step: it also writes the trace
+    hipLaunchKernelGGL(quant_step, grid1d(BH), dim3(kRedThreads), 0, stream, part, np, c, st, a->trace, t, T, 1, out_t,
+                       a->so_b, out_on ? out_t : nullptr, a->so_b, in_on && t + 1 < T ? hq : nullptr, (int64_t)B, H,
+                       out_on ? 1 : 0);
+    GS_CHECK_HIP(hipGetLastError());
+  }
   return GS_OK;
 }
 
@@ -731,8 +821,9 @@ extern "C" int gs_observe_scan(const gs_observe_args* a, hipStream_t stream) {
   float* st = reinterpret_cast<float*>(take(p.st));
   float2* part[2];
   for (float2*& q : part) q = reinterpret_cast<float2*>(take(p.part));
-  float* hpre[2];
-  for (float*& q : hpre) q = reinterpret_cast<float*>(take(p.hpre));
+  float* hpre[2] = {};
+  for (int i = 0; i < (p.three ? 1 : 2); ++i) hpre[i] = reinterpret_cast<float*>(take(p.hpre));
+  float* gh = reinterpret_cast<float*>(take(p.gh));
   float* map = reinterpret_cast<float*>(take(p.map));
   void* map_tmp = take(p.map_tmp);
 
@@ -759,6 +850,8 @@ extern "C" int gs_observe_scan(const gs_observe_args* a, hipStream_t stream) {
                        a->sh0_b, part[1]);
     GS_CHECK_HIP(hipGetLastError());
   }
+
+  if (p.three) return three_launches(a, p, c, W, st, part[1], hpre[0], gh, stream, who);
 
   const unsigned nut = (unsigned)((H + 15) / 16);
   const dim3 grid = p.gemm ? dim3(nut, (unsigned)(p.nwg / nut)) : dim3((unsigned)p.nwg);
@@ -795,13 +888,6 @@ extern "C" int gs_observe_scan(const gs_observe_args* a, hipStream_t stream) {
     hipLaunchKernelGGL(fn, grid, dim3(p.gemm ? 512 : kRedThreads), (size_t)lds, stream, s);
     GS_CHECK_HIP(hipGetLastError());
     np = any_dyn ? (int)p.nwg : 0;
-    if (np > 2 * kMaxParts) {
-      // the workgroups of step t have read part[(t + 1) & 1]
-      hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(1024), 0, stream, part[t & 1], np, part[(t + 1) & 1]);
-      GS_CHECK_HIP(hipGetLastError());
-      std::swap(part[0], part[1]);  // its one pair is the next step's input
-      np = 1;
-    }
   }
   // out[T-1] and the last trace entry
   float* out_t = a->out + (int64_t)(T - 1) * a->so_t;

@@ -567,7 +567,8 @@ int gs_observe_tensor(const gs_observe_tensor_args* args, hipStream_t stream);
 /* The T-step scan with quant_h_in and quant_h_out as observers: at step t,
  * q_in sees h_{t-1} (h0, then out[t-1]; T calls), q_out sees the pre-quant h_t
  * (T calls). Same tensors, strides and hidden-map fields as gs_args; the map
- * is materialized (gs_hidden_map_dense) into the scratch, one launch per step. Forward only. */
+ * is materialized (gs_hidden_map_dense) into the scratch; one launch per step, or three
+ * for large batches. Forward only. */
 typedef struct gs_observe_args {
   int32_t kind;     /* GS_KIND_*                                                    */
   const float* gi;

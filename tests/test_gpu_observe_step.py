@@ -1,8 +1,9 @@
 """The observer scan's one launch per step (observe.hip) at the edges of its
 tiles: 16 units, 16 or 32 rows, K splits of 32-k slices, row ends of every
-length, more partials than a workgroup reads, one quantizer in both places.
-Checked step by step from the kernel's own previous output, as in
-test_gpu_observe.py."""
+length, more partials than a wave's first loads, one quantizer in both places;
+and its three launches per step for large batches. Checked step by step from the
+kernel's own previous output, as in test_gpu_observe.py, and the two forms
+against each other."""
 
 from __future__ import annotations
 
@@ -14,14 +15,15 @@ import torch
 import gru_qat_amd as G
 from oracle import gru_oracle as O
 from parity_util import to_dev
-from test_gpu_observe import _cfg, _codes_match, _quant, _run, _teacher_forced
+from test_gpu_observe import _cfg, _codes_match, _frozen, _quant, _run, _teacher_forced
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("shape", [(3, 2, 1), (3, 2, 3), (3, 17, 6), (3, 15, 33), (2, 33, 127), (2, 16, 130), (2, 3, 517),
                                    (2, 280, 257),     # 32 rows a workgroup
-                                   (2, 2200, 256)])   # 1104 partials: reduced by a launch of their own
+                                   (2, 1500, 256),    # three rounds of workgroups, 752 partials
+                                   (2, 2200, 256)])   # four: three launches a step
 @pytest.mark.parametrize("mode,symmetric", [("min_max", True), ("dynamic", False)])
 def test_observe_step_edges(dev, shape, mode, symmetric):
     cfg = _cfg(1, shape)
@@ -126,3 +128,30 @@ def test_observe_codes_past_24_bits(dev, idx, mode):
     out = _observe_raw(dev, *args, off, q_out)[0].cpu()
     ref = torch.round(pre / s).clamp(-lim, lim) * s
     assert torch.equal(out, ref), f"{int((out != ref).sum())} of {ref.numel()} differ"
+
+
+@pytest.mark.parametrize("shape", [(3, 2100, 100), (2, 8200, 64), (2, 260, 640), (3, 8200, 33), (2, 70, 3072)])
+@pytest.mark.parametrize("q_in,q_out", [(None, None), (0.01, 0.01), (0.02, None), (None, 0.03)])
+def test_observe_three_launches_match_one(dev, shape, q_in, q_out):
+    """Rows of a batch that takes three launches a step equal the same rows alone, which take one."""
+    cfg = _cfg(1, shape)
+    qs = [None if s is None else _frozen(s) for s in (q_in, q_out)]
+    whole, _ = _run(cfg, dev, *qs)
+    for lo in (0, shape[1] - 7):
+        part = dict(cfg, gi=cfg["gi"][:, lo:lo + 7].contiguous(), h0=cfg["h0"][lo:lo + 7].contiguous(), B=7)
+        assert torch.equal(whole[:, lo:lo + 7], _run(part, dev, *qs)[0]), lo
+
+
+def test_observe_batch_past_the_grid(dev):
+    """32-row tiles of 2097121 rows are one more than a grid's second dimension holds."""
+    T, B, H = 2, 32 * 65535 + 1, 2
+    cfg = _cfg(1, (T, B, H))
+    q = _quant("min_max", True).to(dev)
+    out, trace = _run(cfg, dev, q, None)
+    for lo in (0, B - 7):
+        part = dict(cfg, gi=cfg["gi"][:, lo:lo + 7].contiguous(), h0=cfg["h0"][lo:lo + 7].contiguous(), B=7)
+        for t in range(T):  # one step at the whole batch's scale
+            step = dict(part, gi=part["gi"][t:t + 1], h0=part["h0"] if t == 0 else out[t - 1, lo:lo + 7].cpu(), T=1)
+            assert torch.equal(out[t, lo:lo + 7], _run(step, dev, _frozen(float(trace[t, 0])), None)[0][0])
+    scale = torch.stack([cfg["h0"].abs().max(), out[0].abs().max().cpu()]) / 127.0
+    assert torch.equal(trace[:, 0].cpu(), scale)
