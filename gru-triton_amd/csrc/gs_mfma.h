@@ -401,7 +401,8 @@ int run_step_fwd(const gs_args* a, hipStream_t stream, const int8_t* codes, cons
 // Dense shapes that the persistent kernels accept but a launch per step serves
 // faster: B rows give each resident group of workgroups so many 4-row blocks to
 // take in turn every step that the whole batch in one launch is shorter.
-bool step_fwd_beats_persistent(const gs_args* a, bool i8);
+// pack: the persistent kernel would exchange packed levels.
+bool step_fwd_beats_persistent(const gs_args* a, bool i8, bool pack);
 bool step_bwd_beats_persistent(int64_t T, int64_t B, int64_t H);
 bool step_bwd_applies(const float* dout, const float* dh0, int64_t T, int64_t B, int64_t H);
 int run_step_bwd_recurrence(const float* w, float* wt, const float* dout, const float* cg, const float* zm,

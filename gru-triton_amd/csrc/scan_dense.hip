@@ -541,7 +541,8 @@ int run(int kind, const gs_args* a, hipStream_t stream, const char* who, const i
   // every A operand must be a q_in level in the published levels' scale (with q_in on,
   // the packed exchange publishes q_in's levels)
   const bool i8 = codes != nullptr && kind == kDense && dense_i8_applies(a) && pl.pack && a->q_in.scale == pl.pscale;
-  if (kind == kDense && step_fwd_beats_persistent(a, i8)) return run_step_fwd(a, stream, i8 ? codes : nullptr, scales);
+  if (kind == kDense && step_fwd_beats_persistent(a, i8, pl.pack))
+    return run_step_fwd(a, stream, i8 ? codes : nullptr, scales);
   DFn fn = pick(kind, pl.remote, pl.KC, &pl.nt, pl.pack, a->gh_save != nullptr, i8);
   const int threads = 64 * (pl.nwc + (pl.remote ? 4 * pollers_per_row(pl.KC) : 0));
   const int per_set = pl.P * (kind == kMonarch1 ? pl.nb : 1);

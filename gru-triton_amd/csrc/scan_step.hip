@@ -711,19 +711,36 @@ int64_t persistent_rounds(int64_t B, int64_t H, int kc) {
 bool pays_launches(int64_t T, int64_t rounds) { return T == 1 || T * rounds >= 32; }
 }  // namespace
 
-// The persistent kernels take about 1.15 us (H <= 256), 1.5 (<= 512) or 2.8 (<=
-// 1024) a round, int8 codes 0.8, 1.1 or 1.0; a step here 4 to 8 us plus its
-// products. Measured, us a step, persistent / here: fp32 H = 256, B = 256 (4
-// rounds) 4.6 / 4.8, B = 384 (6) 6.7 / 5.5; H = 384, B = 160 (4) 6.9 / 5.3;
-// H = 512, B = 96 (3) 4.7 / 5.7, B = 256 (8) 12.0 / 7.7; H = 640, B = 48 (2) 6.1 / 6.2;
-// H = 1024, B = 48 (3) 8.7 / 8.0, B = 256 (16) 44.3 / 19.6. int8 H = 256, B = 384 (6)
-// 4.5 / 4.4; H = 384, B = 160 (4) 5.1 / 4.1; H = 768, B = 96 (5) 5.9 / 6.5, B = 160 (8) 8.6 /
-// 6.5; H = 1024, B = 160 (10) 9.7 / 11.3, B = 256 (16) 15.2 / 11.7.
-bool step_fwd_beats_persistent(const gs_args* a, bool i8) {
+// The persistent kernels take about 1.2 us (H <= 256), 1.65 (<= 512) or 2.9 (<= 1024)
+// a round, with the packed exchange (pack) 1.3, 1.55 or 2.5, int8 codes 0.8, 1.1 or
+// 1.0; a step here 4 to 8 us plus its products, more where rows are not whole
+// 64-byte lines (H % 16) and where gh is saved along such rows. So each of them moves
+// the number of rounds from which a step here is shorter. Measured at T = 40, us a
+// step, persistent / here: H = 256, B = 384 (6 rounds) 6.7 / 5.5; H = 384, B = 160 (4)
+// 6.8 / 5.4; H = 512, B = 128 (4) 6.2 / 5.9, packed 5.8 / 5.8; H = 500, B = 128 (4) 6.1 / 6.2,
+// B = 160 (5) packed 7.2 / 7.4, packed with gh 7.4 / 8.2; H = 640, B = 72 (3) 8.6 / 6.3;
+// H = 900, B = 48 (3) 8.6 / 7.8, packed 7.6 / 7.8; H = 1000, B = 48 (3) 8.7 / 8.9, packed
+// 7.6 / 8.9, B = 64 (4) packed 10.0 / 11.0, B = 80 (5) packed with gh 12.7 / 12.3; H = 1024,
+// B = 48 (3) 8.7 / 8.0, packed 7.6 / 7.9, B = 256 (16) 44.3 / 19.6. int8 codes: H = 256,
+// B = 384 (6) 4.5 / 4.4; H = 384, B = 160 (4) 5.1 / 4.1; H = 768, B = 96 (5) 5.9 / 6.5,
+// B = 160 (8) 8.6 / 6.5; H = 1024, B = 160 (10) 9.7 / 11.3, B = 256 (16) 15.2 / 11.7.
+static int64_t least_rounds(int64_t H, int kc, bool i8, bool pack, bool save) {
+  if (i8) return kc == 16 ? 7 : kc == 32 ? 4 : H <= 768 ? 7 : 12;
+  if (kc == 16) return 6;
+  const bool lines = H % 16 == 0;
+  if (kc == 32) {
+    if (lines || H <= 320) return 4;
+    return save ? (H <= 384 ? 5 : 6) : H <= 448 ? 4 : pack ? 6 : 5;
+  }
+  if (lines) return pack && H > 896 ? 4 : 3;
+  return H <= (pack || save ? 832 : 928) ? 3 : pack && H > 960 ? 5 : 4;
+}
+
+bool step_fwd_beats_persistent(const gs_args* a, bool i8, bool pack) {
   const int kc = a->H <= kPersistentMaxH ? choose_kc((int)a->H) : 0;
   const int64_t rounds = kc < 16 ? 0 : persistent_rounds(a->B, a->H, kc);
-  const int64_t least = i8 ? (kc == 16 ? 7 : kc == 32 ? 4 : a->H <= 768 ? 7 : 12) : kc == 16 ? 6 : kc == 32 ? 4 : 3;
-  return kc >= 16 && rounds >= least && pays_launches(a->T, rounds) && step_fwd_applies(a);
+  return kc >= 16 && rounds >= least_rounds(a->H, kc, i8, pack, a->gh_save != nullptr) &&
+         pays_launches(a->T, rounds) && step_fwd_applies(a);
 }
 
 // The whole backward, us a step, persistent / here: H = 256, B = 384 (6 rounds)

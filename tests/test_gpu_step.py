@@ -72,7 +72,8 @@ def test_step_int8_codes(dev, shape, q_out):
         assert err <= 1.01 / 127, err
 
 
-@pytest.mark.parametrize("shape", [(11, 48, 1000), (8, 97, 640), (4, 250, 501), (1, 260, 320)])
+# (11, 48, 1000): launches backward only, its forward is a round short of the rule; the others both ways
+@pytest.mark.parametrize("shape", [(11, 48, 1000), (7, 65, 1000), (8, 97, 640), (4, 250, 501), (1, 260, 320)])
 @pytest.mark.parametrize("q", [None, Q_INT8_HIDDEN])
 def test_large_batches_on_the_persistent_entries(dev, shape, q):
     """gru_scan_persistent's batches that run with a launch per step: every row equals the same row of a
