@@ -86,7 +86,7 @@ CASES = [
     ((12, 37, 256), Q_INT8_HIDDEN, Q_INT8_HIDDEN),
     ((7, 3, 80), Q_INT8_HIDDEN, Q_INT8_HIDDEN),
     ((20, 6, 304), Q_INT8_HIDDEN, Q_INT8_HIDDEN),
-    ((6, 5, 1536), Q_INT8_HIDDEN, Q_INT8_HIDDEN),  # H > 1024: the batch-tiled int8 kernel
+    ((6, 5, 1536), Q_INT8_HIDDEN, Q_INT8_HIDDEN),  # H > 1024: one launch per step
     ((5, 3, 2048), Q_INT8_HIDDEN, Q_INT8_HIDDEN),
     ((16, 8, 512), Q_INT8_HIDDEN, None),
     ((16, 8, 512), Q_INT8_HIDDEN, Q_OTHER),
