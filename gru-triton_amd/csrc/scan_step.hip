@@ -699,11 +699,10 @@ bool step_fwd_applies(const gs_args* a) {
 }
 
 namespace {
-// 4-row blocks that a group of the persistent dense kernels takes in turn: P
-// workgroups of 16 units (48 below KC 16) a group, one workgroup per CU.
-int64_t persistent_rounds(int64_t B, int64_t H, int kc) {
-  const int64_t upw = kc >= 16 ? 16 : 48;
-  const int64_t groups = std::max<int64_t>(1, 256 / ((H + upw - 1) / upw));
+// 4-row blocks that a group of the persistent dense kernels (KC 16 and up) takes
+// in turn: one workgroup of 16 units per CU.
+int64_t persistent_rounds(int64_t B, int64_t H) {
+  const int64_t groups = std::max<int64_t>(1, 256 / ((H + 15) / 16));
   return ((B + 3) / 4 + groups - 1) / groups;
 }
 // T launches cost the host 2.5 us each, which shows while the whole recurrence
@@ -738,7 +737,7 @@ static int64_t least_rounds(int64_t H, int kc, bool i8, bool pack, bool save) {
 
 bool step_fwd_beats_persistent(const gs_args* a, bool i8, bool pack) {
   const int kc = a->H <= kPersistentMaxH ? choose_kc((int)a->H) : 0;
-  const int64_t rounds = kc < 16 ? 0 : persistent_rounds(a->B, a->H, kc);
+  const int64_t rounds = kc < 16 ? 0 : persistent_rounds(a->B, a->H);
   return kc >= 16 && rounds >= least_rounds(a->H, kc, i8, pack, a->gh_save != nullptr) &&
          pays_launches(a->T, rounds) && step_fwd_applies(a);
 }
@@ -749,7 +748,7 @@ bool step_fwd_beats_persistent(const gs_args* a, bool i8, bool pack) {
 bool step_bwd_beats_persistent(int64_t T, int64_t B, int64_t H) {
   const int kc = H <= kPersistentMaxH ? choose_kc((int)H) : 0;
   const int64_t least = kc == 16 ? 7 : kc == 32 ? 7 : 3;
-  const int64_t rounds = kc < 16 ? 0 : persistent_rounds(B, H, kc);
+  const int64_t rounds = kc < 16 ? 0 : persistent_rounds(B, H);
   return kc >= 16 && B <= kStepMaxB && rounds >= least && pays_launches(T, rounds);
 }
 
