@@ -53,3 +53,16 @@ def test_size_queries_on_packed_args():
     with pytest.raises(ValueError):
         _lib.raw_size(lib, "gs_input_proj_bwd_workspace_bytes",
                       _lib.PROJ_BWD_ARGS.pack(*([4096] * 7), 0, 0, 0, *rest[1:]))
+
+
+@pytest.mark.parametrize("M,N,I", [(1, 3, 1), (64, 96, 32), (1650, 1503, 301), (4282, 5787, 1929)])
+def test_projection_backward_workspace_kept_by_size(M, N, I):
+    """What the backward keeps per size is the query's answer for its call, quantized or not."""
+    from gru_qat_amd.input_proj import _bwd_workspace_bytes
+
+    for q in (OFF, Q):
+        a = _lib.GsProjBwdArgs(*([4096] * 7), 0, 0, M, N, I, I + 5, N + 7, I, *_quants(q), 4096, 4096, *_quants(q))
+        need = _lib.load().gs_input_proj_bwd_workspace_bytes(ctypes.byref(a))
+        assert _bwd_workspace_bytes(M, N, I) == max(need, 256)
+    with pytest.raises(ValueError):
+        _bwd_workspace_bytes(0, N, I)
