@@ -31,10 +31,11 @@
 // exchange and the epilogue, about 3.3 us a step), then Wh from the caches (12
 // KiB a 64-k chunk and workgroup, 16 KiB with the state), and from a few hundred
 // rows x 1024 units the fp32 MFMA rate: at B = 256, H = 1024 a forward step's
-// products take 12.5 us at the measured 129 TFLOP/s and the step 19.0. Measured us a
-// step, batch-tiled -> here: forward H = 512, B = 32: 59.6 -> 5.9; H = 2048, B = 32:
-// 991 -> 14.6 (int8 codes 364 -> 8.7); whole backward per step: H = 512 37.6 -> 10.9,
-// H = 2048 556 -> 51.8 (of which the products outside the recurrence about 30).
+// products take 12.5 us at the measured 129 TFLOP/s and the step 19.9. Measured us a
+// step, batch-tiled -> here: forward H = 512, B = 32: 59.6 -> 5.4; H = 2048, B = 32:
+// 991 -> 12.6 (int8 codes 364 -> 7.6); whole backward per step: H = 512 37.6 -> 8.9,
+// H = 2048 556 -> 35.0 (23 of it the recurrence); at B = 256, H = 1024 the recurrence takes
+// 28 us a step and the whole backward 56.
 #include "gs_gemm.h"
 #include "gs_mfma.h"
 

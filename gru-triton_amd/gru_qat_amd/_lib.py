@@ -29,7 +29,7 @@ KIND_DIAGONAL = 1
 KIND_MONARCH = 2
 KIND_BUTTERFLY = 3
 KIND_CIRCULANT = 4
-KIND_DENSE_TILED = 5  # size queries of the batch-tiled dense entry points
+KIND_DENSE_TILED = 5  # size queries of the barrier-free dense entry points
 
 # Every symbol include/gruscan.h declares.
 EXPORTS = (

@@ -120,7 +120,8 @@ def gru_scan_forward(
     h_out_quant: QuantTuple = None,
 ) -> torch.Tensor:
     """Same contract as the reference's barrier-free launcher (scan.py:1688-1765):
-    the batch-tiled kernel, no co-residency requirement, any H up to 8192."""
+    one launch per step, or one workgroup per tile of batch rows; no co-residency
+    requirement, any H up to 8192."""
     return _dense_forward("gru_scan_forward", gi, h0, Wh_cat, bh_cat, h_in_quant, h_out_quant, tiled=True,
                           int8_codes=True)
 
@@ -131,8 +132,8 @@ def gru_scan_backward_persistent(gi, h0, Wh_cat, bh_cat, out, dout, *, h_in_quan
 
     Same contract as the reference's gru_scan_backward_persistent
     (scan.py:646-752): ``gs_dense_bwd`` recomputes gh for every step with one
-    GEMM, runs the reverse recurrence as one persistent launch and forms dWh
-    with a second GEMM; dbh comes back as per-row partials summed here.
+    GEMM, runs the reverse recurrence as one persistent launch (for large
+    batches as one launch per step) and forms dWh with a second GEMM; dbh comes back as per-row partials summed here.
     """
     return _dense_backward("gru_scan_backward_persistent", gi, h0, Wh_cat, bh_cat, out, dout, h_in_quant,
                            h_out_quant)
@@ -140,7 +141,7 @@ def gru_scan_backward_persistent(gi, h0, Wh_cat, bh_cat, out, dout, *, h_in_quan
 
 def gru_scan_backward_triton(gi, h0, Wh_cat, bh_cat, out, dout, *, h_in_quant=None, h_out_quant=None):
     """Gradients (dgi, dh0, dWh_cat, dbh_cat) of the dense scan with the
-    reverse recurrence on the barrier-free batch-tiled kernel
+    reverse recurrence on the barrier-free kernels
     (``gs_dense_bwd_tiled``); same contract as the reference's
     gru_scan_backward_triton (scan.py:1355-1447)."""
     return _dense_backward("gru_scan_backward_triton", gi, h0, Wh_cat, bh_cat, out, dout, h_in_quant,
@@ -226,7 +227,7 @@ class GRUScanPersistentFunction(torch.autograd.Function):
 
 
 class GRUScanFunction(torch.autograd.Function):
-    """The same contract on the barrier-free batch-tiled kernels
+    """The same contract on the barrier-free kernels
     (scan.py:1556-1604: the reference's gru_scan Function, whose forward and
     backward are its non-persistent kernels)."""
 
@@ -269,6 +270,6 @@ def gru_scan(
     h_out_quant: QuantTuple = None,
 ) -> torch.Tensor:
     """Differentiable dense GRU scan (reference scan.py:1607-1627) on the
-    barrier-free batch-tiled kernels; returns out [T, B, H]."""
+    barrier-free kernels; returns out [T, B, H]."""
     return cast(torch.Tensor, GRUScanFunction.apply(gi, h0, Wh_cat, bh_cat, h_in_quant, h_out_quant,
                                                     save_gh_default(gi, h0, Wh_cat, bh_cat)))

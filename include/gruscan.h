@@ -83,7 +83,7 @@ extern "C" {
  * weight gradient back onto col. */
 #define GS_KIND_CIRCULANT 4
 /* Size queries only (gs_workspace_bytes, gs_bwd_workspace_bytes, gs_bwd_scratch_bytes): the
- * batch-tiled dense entry points gs_dense_fwd_tiled / gs_dense_bwd_tiled. */
+ * barrier-free dense entry points gs_dense_fwd_tiled / gs_dense_bwd_tiled. */
 #define GS_KIND_DENSE_TILED 5
 
 /* Frozen per-tensor symmetric fake-quant: q = clamp(rint(x / scale), qmin, qmax) * scale,
@@ -164,8 +164,8 @@ int gs_dense_fwd_tiled(const gs_args* args, hipStream_t stream);
 int gs_dense_fwd_i8w(const gs_args* args, const int8_t* w_codes, const float* w_scale, hipStream_t stream);
 
 /* gs_dense_fwd_tiled with the int8 codes of gs_dense_fwd_i8w (reference gru_scan_forward,
- * scan.py:1688-1765, on frozen int8 weights): the batch-tiled kernel reads the codes
- * instead of the fp32 weights every step (a quarter of the bytes) and runs the same
+ * scan.py:1688-1765, on frozen int8 weights): its kernels read the codes instead
+ * of the fp32 weights every step (a quarter of the bytes) and run the same
  * int8 products under the same rule, so it returns gs_dense_fwd_i8w's outputs bit for
  * bit up to H = 1024. No counterpart in the reference beyond that entry point. */
 int gs_dense_fwd_tiled_i8w(const gs_args* args, const int8_t* w_codes, const float* w_scale, hipStream_t stream);
@@ -203,7 +203,7 @@ int gs_butterfly_fwd(const gs_args* args, hipStream_t stream);
  * 2^32 - 2^24 (about 67 million replays of a T = 64 scan), after which tags
  * could repeat. fault_mirror is this entry point's only fault channel:
  * gs_workspace_status cannot reach the static array. Above H = 1024 the
- * batch-tiled kernel runs, which exchanges nothing and uses no array. */
+ * kernels of gs_dense_fwd_tiled run, which exchange nothing and use no array. */
 int gs_dense_fwd_noalloc(const gs_args* args, hipStream_t stream);
 
 /* Same contract as gs_butterfly_fwd, but always runs the general LDS kernel
@@ -295,7 +295,7 @@ int gs_dense_bwd_tiled(const gs_bwd_args* args, hipStream_t stream);
  * 128 and a butterfly with one chain at 2^log_n in {256, 512, 1024} run
  * block-local / stage-wise kernels. Otherwise the hidden map, linear in q_in(h),
  * is materialized as a [3H, H] matrix and run through the dense backward (its
- * recurrence persistent up to H = 1024, batch-tiled beyond), and its [3H, H]
+ * recurrence as gs_dense_bwd's), and its [3H, H]
  * gradient is carried onto the structured parameters (dw_part, and dw2_part for
  * a two-factor Monarch): H <= 8192 for Monarch, 2^log_n <= 4096 for butterfly.
  * The stage-wise butterfly backward runs its twiddle gradient on a stream the
