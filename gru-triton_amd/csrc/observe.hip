@@ -58,8 +58,10 @@ struct ObsPair {
   Obs in, out;
 };
 
+// (Only min_max keeps statistics: elsewhere a stats pointer, which may be the other observer's, is nobody's.)
 Obs to_obs(const gs_observer& o) {
-  return Obs{o.mode, o.symmetric, (float)o.qmin, (float)o.qmax, o.scale, o.zero_point, o.stats};
+  return Obs{o.mode, o.symmetric, (float)o.qmin, (float)o.qmax, o.scale, o.zero_point,
+             o.mode == GS_OBS_MIN_MAX ? o.stats : nullptr};
 }
 
 __host__ __device__ inline bool is_dynamic(const Obs& o) {
@@ -265,8 +267,9 @@ __global__ __launch_bounds__(kRedThreads) void gates_step(const float* gi_t, int
 
 // fq at a scale found at run time. A symmetric one in quant_code's range takes
 // its division-free quotient, which equals the IEEE one (gs_device.h). Codes stay
-// below 2^22 there: the bound under which q_in repeats q_out (same_quant,
+// within kQuickCodes there: the bound under which q_in repeats q_out (same_quant,
 // gs_host.h), inside the 2^24 up to which the quotient holds.
+constexpr int kQuickCodes = 1 << 22;
 struct DynQuant {
   Quant q;
   float zp;
@@ -282,10 +285,12 @@ struct DynQuant {
   }
 };
 
+// WIDE: the range may exceed kQuickCodes.
+template <bool WIDE>
 __device__ __forceinline__ DynQuant dyn_quant(const Obs& o, float s, float zp) {
   DynQuant d{{s, o.qmin, o.qmax, 1, 1.0f / s}, zp, o.mode != GS_OBS_OFF, 0};
-  d.fast = d.on && zp == 0.0f && s >= 0x1p-126f && s <= 0x1p64f && o.qmin >= -0x1p22f &&
-           o.qmax <= 0x1p22f;
+  d.fast = d.on && zp == 0.0f && s >= 0x1p-126f && s <= 0x1p64f;
+  if constexpr (WIDE) d.fast = d.fast && o.qmin >= (float)-kQuickCodes && o.qmax <= (float)kQuickCodes;
   return d;
 }
 
@@ -352,6 +357,7 @@ __device__ __forceinline__ void observe_in(const Obs& o, float (&s)[3], float mn
 // Reduces the partials (each wave by itself: no barrier) and derives the scales
 // of step t: q_out for h_{t-1} (none at t = 0: h0 is not quantized) and q_in.
 // Workgroup 0 updates the statistics, the scale words and the trace.
+template <bool WIDE>
 __device__ __forceinline__ void step_scales(const OStep& p, StepIn& v, DynQuant* qout, DynQuant* qin) {
   float mn = v.part[0].x, mx = v.part[0].y;
 #pragma unroll
@@ -376,7 +382,7 @@ __device__ __forceinline__ void step_scales(const OStep& p, StepIn& v, DynQuant*
       scale_zp(p.c.out, mn, mx, &s_out, &zp_out);
       if (writer) {
         observe_in(p.c.out, v.out, mn, mx);
-        if (p.c.out.mode == GS_OBS_MIN_MAX && p.c.in.stats == p.c.out.stats) {  // one quantizer in both places
+        if (p.c.in.stats == p.c.out.stats) {  // one quantizer in both places
 #pragma unroll
           for (int j = 0; j < 3; ++j) v.in[j] = v.out[j];
         }
@@ -401,9 +407,9 @@ __device__ __forceinline__ void step_scales(const OStep& p, StepIn& v, DynQuant*
       p.st[1] = zp_in;
     }
   }
-  *qout = dyn_quant(p.c.out, s_out, zp_out);
+  *qout = dyn_quant<WIDE>(p.c.out, s_out, zp_out);
   if (p.first) qout->on = qout->fast = 0;
-  *qin = dyn_quant(p.c.in, s_in, zp_in);
+  *qin = dyn_quant<WIDE>(p.c.in, s_in, zp_in);
   // q_in repeats q_out: the levels it sees are its own (same_quant, gs_host.h)
   if (qout->fast && qin->fast && s_in == s_out && p.c.in.qmin == p.c.out.qmin && p.c.in.qmax == p.c.out.qmax)
     qin->on = qin->fast = 0;
@@ -492,7 +498,7 @@ __global__ __launch_bounds__(512) void observe_step_kernel(OStep p) {
   const float hraw = p.hprev[erc * p.sh_b + euc];
 
   DynQuant qout, qin;
-  step_scales(p, in, &qout, &qin);
+  step_scales<false>(p, in, &qout, &qin);
 
   // one division-free quantizer for the state (the common case): applied as the rows are staged
   const bool one_quant = (qout.fast && !qin.on) || (qin.fast && !qout.on);
@@ -599,7 +605,7 @@ __global__ __launch_bounds__(kRedThreads) void observe_diag_kernel(OStep p) {
   __shared__ float2 red2[kRedThreads / 64];
   StepIn in = load_step_in(p);
   DynQuant qout, qin;
-  step_scales(p, in, &qout, &qin);
+  step_scales<true>(p, in, &qout, &qin);
   const int H = p.H;
   float mn = __builtin_inff(), mx = -__builtin_inff();
   const int64_t n = (int64_t)p.B * H;
@@ -683,6 +689,12 @@ bool one_launch(int64_t H, int split, int64_t nwg) {
   return rounds == 2 ? H <= 2048 : rounds == 3 && H >= 192 && H <= 1024;
 }
 
+// Codes past kQuickCodes take three: a check in the one-launch kernel costs every
+// step 0.07 us of its 7.9.
+bool wide_codes(const gs_observer& o) {
+  return o.mode != GS_OBS_OFF && (o.qmin < -kQuickCodes || o.qmax > kQuickCodes);
+}
+
 gs_map_args map_view(const gs_observe_args* a) {
   gs_map_args m{};
   m.kind = a->kind;
@@ -732,7 +744,7 @@ int plan_observe(const gs_observe_args* a, OPlan* p, const char* who) {
   const int64_t nut = (H + 15) / 16;
   p->rt = ((B + 15) / 16) * nut > 256 ? 2 : 1;
   p->nwg = p->gemm ? ((B + 16 * p->rt - 1) / (16 * p->rt)) * nut : parts_for(B * H);
-  p->three = p->gemm && !one_launch(H, p->split, p->nwg);
+  p->three = p->gemm && (wide_codes(a->q_in) || wide_codes(a->q_out) || !one_launch(H, p->split, p->nwg));
   if (p->three) p->nwg = parts_for(B * H);
   p->st = 256;
   p->part = align256(std::max<int64_t>(p->nwg, kMaxParts) * 8);
